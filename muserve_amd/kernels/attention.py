@@ -97,7 +97,7 @@ def attn_prefill_paged(
                     max_seqlen_q, softmax_scale, causal, out, max_seqlen_k)
 
 
-PREFILL_Q_TILE = 32            # query tokens per workgroup of the prefill kernel
+PREFILL_Q_TILE = 64            # query tokens per workgroup of the prefill kernel
 PREFILL_KV_TILE = 64           # keys per step of the prefill kernel (key ranges are multiples)
 PREFILL_SPLIT_MIN = 256        # keys per range at least
 _prefill_ws: dict[torch.device, torch.Tensor] = {}

@@ -326,3 +326,30 @@ def test_one_hot_keys_pin_every_tile_and_split_boundary():
             _bf16_close(rows[:, h], want)
     # rows outside every sequence's queries are left alone by the merge
     assert torch.equal(out[Tq:].view(torch.int16), canary[Tq:])
+
+
+@pytest.mark.parametrize("lens,scale,grow", [
+    ([31, 33, 97], 256 ** -0.5, 0.0),             # 4-wave workgroups: 32-query tiles
+    ([63, 65, 129, 1], -0.07, 0.0),               # a negative scale (queries' signs flip)
+    ([40, 300], 0.0, 0.0),                        # zero: every visible key weighs the same
+    ([64] * 70 + [65, 127, 191], 0.05, 0.0),      # 8-wave workgroups: 64-query tiles
+    ([1300, 700] + [64] * 60, 256 ** -0.5, 3e-3),  # maxima that keep rising
+])
+def test_query_tiles_scales_and_rising_maxima(lens, scale, grow):
+    """Both workgroup sizes at the edges of their query tiles; scales whose
+    sign and zero the kernel handles apart; and keys that grow along the
+    sequence, so that the running maximum moves in every tile."""
+    case(f"attn_prefill tiles: {len(lens)} sequences of {min(lens)}..{max(lens)}, scale {scale}")
+    g, cu = seqs(lens, 71 + len(lens))
+    T = int(cu[-1])
+    pos = torch.cat([torch.arange(n) for n in lens]).float()
+    q = torch.randn(T, 4, 256, generator=g).bfloat16()
+    k = (torch.randn(T, 1, 256, generator=g) * (1.0 + grow * pos[:, None, None])).bfloat16()
+    v = torch.randn(T, 1, 256, generator=g).bfloat16()
+    out = A.attn_prefill(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), cu.to(DEV), max(lens),
+                         max(lens), softmax_scale=scale)
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    want = att.prefill_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(),
+                                 cu.numpy(), scale, True, cu_k=cu.numpy(), stats=True)
+    within(out, want)

@@ -677,16 +677,40 @@ int mkv_prefill_attention_bf16(const void* q, const void* k, const void* v, int6
 
 /*
  * Workspace of mkv_prefill_attention_bf16 with `splits` key ranges (0 for
- * one): with splits > 1 every (query tile, KV head) is cut into ranges of
- * split_len keys (a multiple of 64; the last range runs to the sequence's
- * last key) that separate workgroups attend to, and a second kernel merges
- * their (max, sum, output) per query row and head, writing only the rows of
- * the sequences' queries. That fills the GPU when a step has few, short
- * chunks. With splits > 1 the workspace must be 16-byte aligned and hold
- * these bytes (MKV_E_INVALID otherwise). No reference counterpart.
+ * one): with splits > 1 a (query tile, KV head) that sees more than split_len
+ * keys (a multiple of 64) is cut into equal ranges of at most split_len keys
+ * (longer where `splits` ranges would not reach its last key) that separate
+ * workgroups attend to, and a second kernel merges their (max, sum, output)
+ * per query row and head, writing only the rows of the sequences' queries.
+ * That fills the GPU when a step has few, short chunks. With splits > 1 the
+ * workspace must be 16-byte aligned and hold these bytes (MKV_E_INVALID
+ * otherwise). No reference counterpart.
  */
 int64_t mkv_prefill_attention_workspace_bytes(int64_t num_q_tokens, int32_t num_q_heads,
                                               int32_t splits);
+
+/*
+ * mkv_prefill_attention_bf16 with its schedule planned on the device: a first
+ * kernel reads the lengths, chooses how many keys a range holds (at most
+ * `splits` ranges per query tile) and lists the (query tile, KV head, range)
+ * tasks, longest first; the attention and merge kernels follow the list. For
+ * sequences of different lengths and chunks on long prefixes. At most 1024
+ * sequences and 4096 query tiles of 64 times KV heads (tiles: the longest
+ * sequence's times the batch, or num_q_tokens / 64 + batch if that is less;
+ * MKV_E_UNSUPPORTED past them). The workspace (16-byte aligned) holds
+ * mkv_prefill_attention_plan_bytes (-1: unsupported). No reference
+ * counterpart.
+ */
+int mkv_prefill_attention_planned_bf16(
+    const void* q, const void* k, const void* v, int64_t kv_units, int32_t num_kv_heads,
+    int32_t num_q_heads, int32_t head_dim, const int32_t* page_table, int64_t table_stride,
+    int32_t table_width, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+    const int32_t* seq_lens_k, int32_t batch, int64_t num_q_tokens, int32_t max_seqlen_q,
+    float softmax_scale, int32_t causal, int32_t splits, void* out, void* workspace,
+    int64_t workspace_bytes, int32_t* err, void* stream);
+int64_t mkv_prefill_attention_plan_bytes(int64_t num_q_tokens, int32_t num_q_heads,
+                                         int32_t num_kv_heads, int32_t batch,
+                                         int32_t max_seqlen_q, int32_t splits);
 
 /*
  * On-device check of what the fp8 kernels rely on. Adds into counts[7]

@@ -77,6 +77,10 @@ SIGNATURES: dict[str, list] = {
                                    _P, _I32, _I64, _I32, _F32, _I32, _I32, _I32, _P, _P, _I64,
                                    _P, _P],
     "mkv_prefill_attention_workspace_bytes": [_I64, _I32, _I32],
+    "mkv_prefill_attention_planned_bf16": [_P, _P, _P, _I64, _I32, _I32, _I32, _P, _I64, _I32, _P,
+                                           _P, _P, _I32, _I64, _I32, _F32, _I32, _I32, _P, _P,
+                                           _I64, _P, _P],
+    "mkv_prefill_attention_plan_bytes": [_I64, _I32, _I32, _I32, _I32, _I32],
     "mkv_check_conversions": [_P, _P],
     "mkv_bm_state_bytes": [_I32],
     "mkv_bm_layout": [_I32, _P],
@@ -104,7 +108,7 @@ SIGNATURES: dict[str, list] = {
     "mkv_probe_fill": [_P, _I64, _P],
 }
 _INT64_RESULT = {"mkv_bm_state_bytes", "mkv_decode_attention_workspace_bytes",
-                 "mkv_prefill_attention_workspace_bytes"}
+                 "mkv_prefill_attention_workspace_bytes", "mkv_prefill_attention_plan_bytes"}
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None

@@ -29,12 +29,17 @@
 // What bounds it: a K or V byte read from LDS feeds 32 query rows, so a tile
 // is 4096 cycles of a CU's matrix cores against 512 KiB of LDS reads; with 16
 // rows per wave (v_mfma_f32_16x16x32_bf16, P through LDS, tiles through
-// registers) the LDS reads and the passes of P bounded it. On MI355X, 8 x 4096
-// causal tokens of one KV head: 560 -> 380 us (0.49 -> 0.72 PFLOP/s of the
-// visible pairs); two 1.3k-token chunks on 3-5k-token prefixes with their
-// append and merge: 156 -> 80 us. While a CU is busy its matrix cores are so
-// 60 % of the time.
+// registers) the LDS reads and the passes of P bounded it, 560 us against
+// 380 us for 8 x 4096 causal tokens of one KV head on MI355X. What then set
+// the time was which CU ran which tile: workgroups are dealt to the 8 XCDs in
+// turn, and with a sequence's tiles in consecutive workgroups an XCD had 113
+// key tiles on its fullest CU against 65 on average. With the order below
+// (prefill_attn_kernel) the same launch takes 254-262 us (1.05-1.08 PFLOP/s
+// of the visible pairs); six prompts of 80 to 4096 tokens, planned on the
+// device (prefill_plan_kernel), 177 -> 143 us. While a CU is busy its matrix
+// cores are so 59 % of the time, at 1.9 GHz.
 #include <float.h>
+#include <limits.h>
 #include <math.h>
 
 #include "mkv_device.h"
@@ -69,6 +74,27 @@ constexpr int kQTok = 64;          // query tokens per workgroup of 8 waves
 constexpr int kKvTile = 64;        // KV tokens per step
 constexpr int kTileB = kKvTile * kPRow;     // bytes of one staged K (or V) tile
 constexpr int kCus = 256;          // MI355X; LDS holds one workgroup per CU
+constexpr int kXcds = 8;           // MI355X: workgroups go round robin over 8 XCDs
+
+// One workgroup's task of a planned launch: range z of p of the query tile
+// from query qt of a sequence, for KV head hk (zp = z + 65536 p).
+struct PlanItem {
+  int32_t qs, nq, kbase, nk;
+  int32_t b, hk, qt;
+  uint32_t zp;
+};
+static_assert(sizeof(PlanItem) == 32, "two 16-byte loads");
+struct Plan {
+  int32_t items, cuts;  // tasks; (query tile, KV head) pairs of several ranges
+  int32_t pad[14];
+};
+constexpr int kPlanThreads = 1024, kPlanSmall = 256;  // (the small form: quicker barriers)
+constexpr int kPlanSlots = 4;                          // query tiles per thread
+constexpr int kPlanTiles = kPlanThreads * kPlanSlots;  // query tiles at most
+constexpr int kPlanSeqs = kPlanThreads;                // sequences at most
+static_assert(kCus <= kPlanSmall, "tasks that run at once have a bin each, and a tile per thread");
+constexpr int kPlanLeast = 2;                          // key tiles per range at least
+constexpr int kPlanTries = 16;                         // range lengths that a plan tries
 
 struct PrefillArgs {
   const uint8_t* q;      // [Tq, Hq, 256] bf16
@@ -86,8 +112,15 @@ struct PrefillArgs {
   uint8_t* out;          // [Tq, Hq, 256] bf16
   int32_t hkv;
   int32_t causal;
-  int32_t splits;        // key ranges per (query tile, KV head); 1: output directly
-  int32_t split_len;     // keys per range (a multiple of the KV tile)
+  int32_t tok;           // query tokens per workgroup of this launch
+  uint32_t ranks;        // query tiles of the longest sequence the launch covers
+  uint32_t rank0;        // the first tile rank of this launch
+  int32_t splits;        // key ranges per (query tile, KV head) at most
+  int32_t split_len;     // keys a range aims at (a multiple of the KV tile)
+  Plan* plan;            // null: the grid is the schedule
+  PlanItem* items;       // the plan's tasks, longest first
+  PlanItem* cut;         // its pairs of several ranges (z unused)
+  int32_t max_items, max_cuts;
   float* part;           // splits > 1: [Tq, Hq, splits, 256] unnormalised outputs
   float* ml;             // splits > 1: [Tq, Hq, splits, 2] (max, sum), log2 units
   float scale_log2;      // |softmax scale| * log2(e), positive
@@ -119,6 +152,64 @@ __device__ __forceinline__ float half_max(float x) {
 __device__ __forceinline__ float half_sum(float x) {
   const float2 y = both_halves(x);
   return y.x + y.y;
+}
+
+// The queries of sequence b, from row qs: offsets outside the buffer, or more
+// queries than the launch covers, are bad; nothing of the sequence (or nothing
+// past the bound) is touched.
+__device__ __forceinline__ int32_t seq_queries(const PrefillArgs& a, int64_t b, int32_t& qs,
+                                               bool& bad) {
+  qs = a.cu_q[b];
+  const int32_t n = a.cu_q[b + 1] - qs;
+  const bool ok = qs >= 0 && n >= 0 && (int64_t)qs + n <= a.num_q;
+  bad = !ok || n > a.max_q;
+  return ok ? (n < a.max_q ? n : a.max_q) : 0;
+}
+
+// The keys of sequence b: a length checked against what the table (or the
+// buffer) holds; a bad one is flagged and clamped.
+__device__ __forceinline__ int64_t seq_keys(const PrefillArgs& a, int64_t b, int64_t& kbase,
+                                            bool& bad) {
+  int64_t nk;
+  kbase = 0;
+  bad = false;
+  if (a.table) {
+    nk = a.lens_k[b];
+    const int64_t cap = (int64_t)a.twidth * 16;
+    if (nk < 0 || nk > cap) {
+      bad = true;
+      nk = nk < 0 ? 0 : cap;
+    }
+  } else {
+    kbase = a.cu_k[b];
+    nk = (int64_t)a.cu_k[b + 1] - kbase;
+    if (kbase < 0 || nk < 0 || kbase + nk > a.kv_units) {
+      bad = true;
+      nk = 0;
+    }
+  }
+  return nk;
+}
+
+// The end of the keys that the query tile from qt sees (0: none).
+__device__ __forceinline__ int64_t tile_end(const PrefillArgs& a, int64_t nk, int32_t nq,
+                                            int32_t qt) {
+  if (!a.causal) return nk;
+  const int32_t last_q = (qt + a.tok < nq ? qt + a.tok : nq) - 1;
+  const int64_t end = nk - nq + last_q + 1;  // <= nk
+  return end > 0 ? end : 0;
+}
+
+// Key ranges of a query tile that sees `units` key tiles: as many as keep a
+// range at `cap` key tiles, at most the launch's count. Range z of p covers
+// the key tiles from units * z / p to units * (z + 1) / p. A query tile of one
+// range is written by its workgroup, with no partial rows and no merge.
+__device__ __forceinline__ int32_t tile_ranges(int32_t units, int32_t cap, int32_t splits) {
+  const int32_t p = (units + cap - 1) / cap;
+  return p > splits ? splits : p < 1 ? 1 : p;
+}
+__device__ __forceinline__ int32_t units_of(int64_t keys) {
+  return (int32_t)((keys + kKvTile - 1) / kKvTile);
 }
 
 // 16 bytes per lane from base + voff into LDS at lds + 16 * lane. Issued from
@@ -162,52 +253,60 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int n = lane & 31, hf = lane >> 5;
-  const int64_t b = blockIdx.y, hk = blockIdx.z / a.splits, split = blockIdx.z % a.splits;
-  const int32_t qs = a.cu_q[b];
-  const int32_t nq_raw = a.cu_q[b + 1] - qs;
-  // query offsets outside the buffer, or more queries than the launch covers:
-  // flagged; nothing of the sequence (or nothing past the bound) is touched
-  const bool q_ok = qs >= 0 && nq_raw >= 0 && (int64_t)qs + nq_raw <= a.num_q;
-  if ((!q_ok || nq_raw > a.max_q) && tid == 0 && blockIdx.x == 0 && blockIdx.z == 0)
-    raise_err(a.err, MKV_DEVERR_TABLE);
-  const int32_t nq = q_ok ? (nq_raw < a.max_q ? nq_raw : a.max_q) : 0;
-  // the workgroup's first query; a causal sequence's last tiles see the most
-  // keys and start first
-  const int32_t qt = (int32_t)(gridDim.x - 1 - blockIdx.x) * kTok;
-  if (qt >= nq) return;  // uniform
+  int64_t b, hk, kbase, nk;
+  int32_t qs, nq, qt, split, ranges;
+  if (a.plan) {
+    if ((int32_t)blockIdx.x >= ld_const(&a.plan->items)) return;  // uniform
+    const PlanItem* it = a.items + blockIdx.x;
+    qs = ld_const(&it->qs);
+    nq = ld_const(&it->nq);
+    kbase = ld_const(&it->kbase);
+    nk = ld_const(&it->nk);
+    b = ld_const(&it->b);
+    hk = ld_const(&it->hk);
+    qt = ld_const(&it->qt);
+    const uint32_t zp = (uint32_t)ld_const(reinterpret_cast<const int32_t*>(&it->zp));
+    split = (int32_t)(zp & 0xffffu);
+    ranges = (int32_t)(zp >> 16);
+    if (ranges == 0) return;  // uniform: a gap in the list
+  } else {
+    // Workgroups come in the order of their tile's rank, the sequences' last
+    // tiles (which see the most keys, if causal) first, and all (sequence, KV
+    // head, range) triples of a rank before the next rank. The dispatcher
+    // hands consecutive workgroups to the 8 XCDs in turn, whatever their
+    // load, so a triple moves one XCD on with every 8 workgroups: each XCD
+    // gets tiles of all ranks of every sequence.
+    const uint32_t triples = gridDim.x * gridDim.y;
+    const uint32_t rank = a.rank0 + blockIdx.z;
+    const uint64_t turn = triples >= kXcds ? rank : (uint64_t)rank * triples / kXcds;
+    uint32_t at = (uint32_t)(((uint64_t)blockIdx.y * gridDim.x + blockIdx.x + turn) % triples);
+    split = (int32_t)(at % (uint32_t)a.splits);
+    at /= (uint32_t)a.splits;
+    b = at / (uint32_t)a.hkv;
+    hk = at % (uint32_t)a.hkv;
+    bool bad;
+    nq = seq_queries(a, b, qs, bad);
+    if (bad && tid == 0 && rank == 0 && split == 0 && hk == 0) raise_err(a.err, MKV_DEVERR_TABLE);
+    const int64_t q = (int64_t)(a.ranks - 1 - rank) * kTok;  // the workgroup's first query
+    if (q >= nq) return;  // uniform
+    qt = (int32_t)q;
+    nk = seq_keys(a, b, kbase, bad);
+    if (bad && tid == 0 && qt == 0) raise_err(a.err, MKV_DEVERR_TABLE);
+    ranges = tile_ranges(units_of(tile_end(a, nk, nq, qt)), a.split_len / kKvTile, a.splits);
+    if (split >= ranges) return;  // uniform
+  }
   const int64_t hq = (int64_t)a.hkv * kPG;
   const int64_t h = hk * kPG + (wave & 3);      // this wave's query head
   const int32_t q0 = qt + kWTok * (wave >> 2);  // this wave's first query
 
-  // the sequence's keys: a length checked against what the table (or the
-  // buffer) holds; a bad one is flagged and clamped
-  int64_t nk, kbase = 0;
-  bool bad = false;
-  if (a.table) {
-    nk = a.lens_k[b];
-    const int64_t cap = (int64_t)a.twidth * 16;
-    if (nk < 0 || nk > cap) {
-      bad = true;
-      nk = nk < 0 ? 0 : cap;
-    }
-  } else {
-    kbase = a.cu_k[b];
-    nk = (int64_t)a.cu_k[b + 1] - kbase;
-    if (kbase < 0 || nk < 0 || kbase + nk > a.kv_units) {
-      bad = true;
-      nk = 0;
-    }
-  }
-  if (bad && tid == 0 && qt == 0) raise_err(a.err, MKV_DEVERR_TABLE);
   const int64_t shift = nk - nq;  // query t sits at position shift + t
-  const int32_t last_q = (qt + kTok < nq ? qt + kTok : nq) - 1;  // the workgroup's last
-  int64_t kv_end = a.causal ? shift + last_q + 1 : nk;
-  if (kv_end > nk) kv_end = nk;
-  // this workgroup's key range (the whole range with one split); the last
-  // range runs to the sequence's end, so a split_len * splits below the real
-  // key count never drops keys
-  const int64_t kv_begin = split * (int64_t)a.split_len;
-  if (split + 1 < a.splits && kv_begin + a.split_len < kv_end) kv_end = kv_begin + a.split_len;
+  // this workgroup's key range
+  int64_t kv_end = tile_end(a, nk, nq, qt), kv_begin = 0;
+  if (ranges > 1) {
+    const int64_t units = units_of(kv_end);
+    kv_begin = units * split / ranges * kKvTile;
+    if (split + 1 < ranges) kv_end = units * (split + 1) / ranges * kKvTile;
+  }
   // the last key any of this wave's queries sees (-1: it has none), and the
   // last one that all of them see
   int64_t wlast = -1, wfull = -1;
@@ -462,7 +561,7 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
   const int64_t row0 = ((int64_t)qs + q0) * hq + h;
-  if (a.splits == 1) {
+  if (ranges == 1) {
     const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -505,7 +604,8 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
 // dims (16-byte loads of the fp32 partial rows). It writes exactly the rows
 // the attention kernel wrote ranges for: the same query offsets and bounds
 // decide, so rows of `out` outside every sequence's queries are left alone,
-// as with one range. Each output element is summed over the ranges in range
+// as with one range; rows of a tile of one range are already there. Each
+// output element is summed over the ranges in range
 // order, as a thread per element did (one workgroup per query head was 4x
 // the workgroups for the same bytes). Up to 8 ranges, every load
 // is issued before the first is used (a loop over the ranges waited a round
@@ -534,21 +634,37 @@ __device__ __forceinline__ void merge_ranges(const float2* ml, const float* part
 }
 
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
-  const int32_t b = blockIdx.y;
-  const int32_t qs = a.cu_q[b];
-  const int32_t nq_raw = a.cu_q[b + 1] - qs;
-  const bool q_ok = qs >= 0 && nq_raw >= 0 && (int64_t)qs + nq_raw <= a.num_q;
-  const int32_t nq = q_ok ? (nq_raw < a.max_q ? nq_raw : a.max_q) : 0;
-  const int32_t t = blockIdx.x;
-  if (t >= nq) return;
+  int32_t qs, t, ranges;
+  int64_t hk;
+  if (a.plan) {
+    if ((int32_t)blockIdx.y >= ld_const(&a.plan->cuts)) return;
+    const PlanItem* it = a.cut + blockIdx.y;
+    qs = ld_const(&it->qs);
+    hk = ld_const(&it->hk);
+    t = ld_const(&it->qt) + (int32_t)blockIdx.x;
+    if (t >= ld_const(&it->nq)) return;
+    ranges = ld_const(reinterpret_cast<const int32_t*>(&it->zp)) >> 16;
+  } else {
+    const int32_t b = blockIdx.y;
+    int64_t kbase;
+    bool bad;
+    const int32_t nq = seq_queries(a, b, qs, bad);
+    t = blockIdx.x;
+    hk = blockIdx.z;
+    if (t >= nq) return;
+    const int64_t nk = seq_keys(a, b, kbase, bad);
+    ranges = tile_ranges(units_of(tile_end(a, nk, nq, t / a.tok * a.tok)),
+                         a.split_len / kKvTile, a.splits);
+    if (ranges == 1) return;
+  }
   const int64_t row = ((int64_t)qs + t) * ((int64_t)a.hkv * kPG) +
-                      (int64_t)blockIdx.z * kPG + (threadIdx.x >> 6);
+                      hk * kPG + (threadIdx.x >> 6);
   const int d = (threadIdx.x & 63) * 4;
   const int64_t at0 = row * a.splits;
   float O[4] = {0.f, 0.f, 0.f, 0.f}, L = 0.f;
   const float2* ml = reinterpret_cast<const float2*>(a.ml) + at0;
   const float* part = a.part + at0 * kPD + d;
-  switch (a.splits) {
+  switch (ranges) {
     case 2: merge_ranges<2>(ml, part, L, O); break;
     case 3: merge_ranges<3>(ml, part, L, O); break;
     case 4: merge_ranges<4>(ml, part, L, O); break;
@@ -558,8 +674,8 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     case 8: merge_ranges<8>(ml, part, L, O); break;
     default: {  // more than 8 ranges
       float M = -INFINITY;
-      for (int sp = 0; sp < a.splits; ++sp) M = fmaxf(M, a.ml[(at0 + sp) * 2]);
-      for (int sp = 0; sp < a.splits; ++sp) {
+      for (int sp = 0; sp < ranges; ++sp) M = fmaxf(M, a.ml[(at0 + sp) * 2]);
+      for (int sp = 0; sp < ranges; ++sp) {
         const float m = a.ml[(at0 + sp) * 2];
         const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
         const f32x4 p = *reinterpret_cast<const f32x4*>(a.part + (at0 + sp) * kPD + d);
@@ -577,6 +693,246 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   *reinterpret_cast<uint2*>(a.out + row * kPRow + d * 2) = uint2{w[0], w[1]};
 }
 
+// The plan of a launch: the (query tile, KV head, key range) tasks, longest
+// first, and the pairs of several ranges for the merge. A CU runs one
+// workgroup at a time, a key tile after the other, so what decides a launch is
+// the most key tiles that any CU gets. Key tiles per range:
+//   * the fewest with which all tasks run at once, one per CU, if that is not
+//     far above the key tiles per CU (1.5 times + 2);
+//   * else 1.2 times the key tiles per CU: the longest tasks start first, and
+//     the shorter ones fill the CUs as they come free.
+// Only the lengths on the device say which, and a grid sized on the host has
+// workgroups with nothing to do among the others, which leaves some XCD with
+// more tasks than CUs (two 1.3k-token chunks on 3-5k tokens: attention kernel
+// 107 us with a dense grid of 7 ranges, 64 us planned; sorted by length alone,
+// without the XCDs' grouping, 66 us). The plan takes 7-8 us.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void prefill_plan_kernel(PrefillArgs a, int32_t batch) {
+  __shared__ int32_t pre[THREADS];          // the sequences' first tiles
+  __shared__ int4 seq[THREADS];             // qs, nq, kbase, nk
+  __shared__ int32_t bins[THREADS];         // tasks by their key tiles, then where they start
+  __shared__ int32_t red[THREADS / 64][2];
+  __shared__ uint16_t tile_units[THREADS];  // of the first tiles, for the search
+  __shared__ int2 group[THREADS];           // a sequence's first bin, ranges of its last tile
+  __shared__ int32_t cuts, found;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int kWaves = THREADS / 64;
+  // the exclusive prefix of x over the workgroup, and the total
+  auto block_scan = [&](int32_t x, int32_t& total) __attribute__((always_inline)) {
+    int32_t incl = x;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t o = __shfl_up(incl, d);
+      if (lane >= d) incl += o;
+    }
+    __syncthreads();  // red's earlier readers are done
+    if (lane == 63) red[wave][0] = incl;
+    __syncthreads();
+    int32_t at = incl - x;
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      at += w < wave ? red[w][0] : 0;
+      total += red[w][0];
+    }
+    return at;
+  };
+  int32_t mine = 0;
+  if (tid < batch) {
+    int32_t qs;
+    int64_t kbase;
+    bool bad_q, bad_k;
+    const int32_t nq = seq_queries(a, tid, qs, bad_q);
+    const int64_t nk = seq_keys(a, tid, kbase, bad_k);
+    if (bad_q || (bad_k && nq > 0)) raise_err(a.err, MKV_DEVERR_TABLE);
+    seq[tid] = int4{qs, nq, (int32_t)kbase, (int32_t)nk};
+    mine = (nq + kQTok - 1) / kQTok;
+  }
+  bins[tid] = 0;
+  if (tid == 0) {
+    cuts = 0;
+    found = INT_MAX;
+  }
+  int32_t tiles;
+  const int32_t first = block_scan(mine, tiles);
+  pre[tid] = first;  // (sequences past the batch repeat the total)
+  // offsets that overlap (flagged above: some count is then negative) can
+  // hold more tiles than the launch's bound; the ones past it are dropped
+  if (tiles > (THREADS * kPlanSlots)) tiles = (THREADS * kPlanSlots);
+  __syncthreads();
+
+  int32_t sq[kPlanSlots], unit[kPlanSlots];
+  int32_t sum = 0, most = 0;
+#pragma unroll
+  for (int k = 0; k < kPlanSlots; ++k) {
+    const int32_t i = tid + k * THREADS;
+    sq[k] = -1;
+    unit[k] = 0;
+    if (i >= tiles) continue;
+    int lo = 0, hi = batch - 1;  // the last sequence that starts at or before tile i
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (pre[mid] <= i) lo = mid; else hi = mid - 1;
+    }
+    sq[k] = lo;
+    const int4 x = seq[lo];
+    // (as many as 16 bits hold: past 4 M keys the split needs no more)
+    unit[k] = units_of(tile_end(a, x.w, x.y, (i - pre[lo]) * kQTok));
+    unit[k] = unit[k] < 65535 ? unit[k] : 65535;
+    if (k == 0) tile_units[tid] = (uint16_t)unit[k];
+    sum += unit[k];
+    most = unit[k] > most ? unit[k] : most;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    sum += __shfl_xor(sum, d);
+    const int32_t o = __shfl_xor(most, d);
+    most = o > most ? o : most;
+  }
+  if (lane == 0) {  // (red's earlier readers passed the barrier above)
+    red[wave][0] = sum;
+    red[wave][1] = most;
+  }
+  __syncthreads();
+  sum = 0;
+  most = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    sum += red[w][0];
+    most = red[w][1] > most ? red[w][1] : most;
+  }
+  const uint64_t all = (uint64_t)(uint32_t)sum * (uint32_t)a.hkv;  // key tiles of all tasks
+  // key tiles per range: no less than the key tiles per CU (so the tasks are
+  // at most the query tiles and one more per CU) and than the launch's bound
+  int32_t least = (int32_t)((all + kCus - 1) / kCus);
+  const int32_t bound = a.splits > 1 ? (most + a.splits - 1) / a.splits : most;
+  least = least < bound ? bound : least;
+  least = least < kPlanLeast ? kPlanLeast : least;
+  int32_t cap = most;
+  if (a.splits > 1 && least < most) {
+    cap = (int32_t)((all + all / 5 + kCus - 1) / kCus);
+    cap = cap < least ? least : cap > most ? most : cap;
+    // kPlanTries candidates, evenly from the least to `far`
+    int32_t far = (int32_t)(all * 3 / (2 * kCus)) + 2;
+    far = far < least ? least : far > most ? most : far;
+    if ((int64_t)tiles * a.hkv <= kCus) {  // (so tile_units holds them all)
+      const int32_t step = (far - least + kPlanTries - 1) / kPlanTries;
+      for (int c = wave; c < kPlanTries; c += kWaves) {
+        int32_t tried = least + c * (step > 1 ? step : 1);
+        tried = tried < far && c + 1 < kPlanTries ? tried : far;
+        int32_t n = 0;
+        for (int i = lane; i < tiles; i += 64) n += tile_ranges(tile_units[i], tried, a.splits);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d);
+        if (lane == 0 && (int64_t)n * a.hkv <= kCus) atomicMin(&found, tried);
+      }
+      __syncthreads();
+      if (found != INT_MAX) cap = found;
+    }
+  }
+  if (cap < 1) cap = 1;
+
+  // A counting sort of the tasks. All running at once: by (sequence, KV head,
+  // range), each XCD taking a contiguous eighth (workgroup w runs on XCD
+  // w % 8), so that the query tiles reading the same keys share an L2.
+  // Else by key tiles, the longest first.
+  const bool once = found != INT_MAX;  // uniform
+  if (once) {
+    int32_t keys = 0, most_p = 0, unused;
+    if (tid < batch && seq[tid].y > 0) {
+      const int32_t u = units_of(seq[tid].w);  // its last tile's
+      most_p = tile_ranges(u < 65535 ? u : 65535, cap, a.splits);
+      keys = most_p * a.hkv;
+    }
+    const int32_t base = block_scan(keys, unused);
+    group[tid] = int2{base, most_p};
+    __syncthreads();
+  }
+  // the task's bin; consecutive tasks of a tile share one unless `once`
+  auto bin_of = [&](int k, int32_t p, int32_t hk, int32_t z) __attribute__((always_inline)) {
+    if (once) {
+      const int2 g = group[sq[k]];
+      return g.x + hk * g.y + z;
+    }
+    const int32_t len = (unit[k] + p - 1) / p;
+    return THREADS - 1 - (len < THREADS ? len : THREADS - 1);
+  };
+#pragma unroll
+  for (int k = 0; k < kPlanSlots; ++k) {
+    if (sq[k] < 0) continue;
+    const int32_t p = tile_ranges(unit[k], cap, a.splits);
+    if (once) {
+      for (int32_t hk = 0; hk < a.hkv; ++hk)
+        for (int32_t z = 0; z < p; ++z) atomicAdd(&bins[bin_of(k, p, hk, z)], 1);
+    } else {
+      atomicAdd(&bins[bin_of(k, p, 0, 0)], p * a.hkv);
+    }
+  }
+  __syncthreads();
+  int32_t total;
+  const int32_t start = block_scan(bins[tid], total);
+  bins[tid] = start;  // (each thread rewrites the entry that it alone read)
+  __syncthreads();
+  const int32_t per = (total + kXcds - 1) / kXcds;  // tasks per XCD
+  auto place = [&](int32_t at) __attribute__((always_inline)) {
+    return once ? at % per * kXcds + at / per : at;
+  };
+#pragma unroll
+  for (int k = 0; k < kPlanSlots; ++k) {
+    if (sq[k] < 0) continue;
+    const int32_t p = tile_ranges(unit[k], cap, a.splits);
+    const int4 x = seq[sq[k]];
+    const int32_t qt = (tid + k * THREADS - pre[sq[k]]) * kQTok;
+    int32_t at = once ? 0 : atomicAdd(&bins[bin_of(k, p, 0, 0)], p * a.hkv);
+    int32_t c = p > 1 ? atomicAdd(&cuts, a.hkv) : 0;
+    for (int32_t hk = 0; hk < a.hkv; ++hk) {
+      PlanItem it = {x.x, x.y, x.z, x.w, sq[k], hk, qt, (uint32_t)p << 16};
+      if (p > 1) {
+        if (c < a.max_cuts) a.cut[c] = it;
+        ++c;
+      }
+      for (int32_t z = 0; z < p; ++z) {
+        it.zp = ((uint32_t)p << 16) | (uint32_t)z;
+        const int32_t to = place(once ? atomicAdd(&bins[bin_of(k, p, hk, z)], 1) : at++);
+        if (to < a.max_items) a.items[to] = it;
+      }
+    }
+  }
+  if (once && tid < per * kXcds - total) {  // the gaps
+    const int32_t to = place(total + tid);
+    if (to < a.max_items) a.items[to] = PlanItem{0, 0, 0, 0, 0, 0, 0, 0u};
+  }
+  if (once) total = per * kXcds;
+  __syncthreads();
+  if (tid == 0) {
+    a.plan->items = total < a.max_items ? total : a.max_items;
+    a.plan->cuts = cuts < a.max_cuts ? cuts : a.max_cuts;
+  }
+}
+
+inline int64_t align16(int64_t n) { return (n + 15) / 16 * 16; }
+
+// Sizes of a planned launch, from what the host knows: query tiles are
+// bounded by the longest sequence's times the batch, and by the rows.
+struct PlanSizes {
+  int64_t tiles, items, cuts, bytes;
+};
+inline PlanSizes plan_sizes(int64_t num_q, int32_t hkv, int32_t batch, int32_t max_q,
+                            int32_t splits, int32_t cus) {
+  PlanSizes s;
+  const int64_t dense = ((int64_t)max_q + kQTok - 1) / kQTok * batch;
+  const int64_t rows = num_q / kQTok + batch;
+  s.tiles = dense < rows ? dense : rows;
+  // a range is no shorter than the key tiles per CU, so cutting adds at most
+  // one task per CU, and at most that many pairs are cut
+  const int64_t pairs = s.tiles * hkv;
+  s.items = pairs * splits < pairs + cus ? pairs * splits : pairs + cus;
+  s.items = (s.items + kXcds - 1) / kXcds * kXcds;  // with the gaps of a list dealt to the XCDs
+  s.cuts = splits == 1 ? 0 : pairs < cus ? pairs : cus;
+  s.bytes = (int64_t)sizeof(Plan) + (s.items + s.cuts) * (int64_t)sizeof(PlanItem);
+  return s;
+}
+
 }  // namespace
 }  // namespace mkv
 
@@ -589,43 +945,50 @@ extern "C" int64_t mkv_prefill_attention_workspace_bytes(int64_t num_q_tokens, i
   return num_q_tokens * num_q_heads * splits * (kPD + 2) * 4;
 }
 
-extern "C" int mkv_prefill_attention_bf16(const void* q, const void* k, const void* v,
-                                          int64_t kv_units, int32_t num_kv_heads,
-                                          int32_t num_q_heads, int32_t head_dim,
-                                          const int32_t* page_table, int64_t table_stride,
-                                          int32_t table_width, const int32_t* cu_seqlens_q,
-                                          const int32_t* cu_seqlens_k, const int32_t* seq_lens_k,
-                                          int32_t batch, int64_t num_q_tokens, int32_t max_seqlen_q,
-                                          float softmax_scale, int32_t causal, int32_t splits,
-                                          int32_t split_len, void* out, void* workspace,
-                                          int64_t workspace_bytes, int32_t* err, void* stream) {
+namespace {
+
+// Shared by the entry points: `planned` launches take their schedule from the
+// plan kernel (split_len unused), others from the grid.
+int prefill_attention(const char* fn, bool planned, const void* q, const void* k, const void* v,
+                      int64_t kv_units, int32_t num_kv_heads, int32_t num_q_heads,
+                      int32_t head_dim, const int32_t* page_table, int64_t table_stride,
+                      int32_t table_width, const int32_t* cu_seqlens_q,
+                      const int32_t* cu_seqlens_k, const int32_t* seq_lens_k, int32_t batch,
+                      int64_t num_q_tokens, int32_t max_seqlen_q, float softmax_scale,
+                      int32_t causal, int32_t splits, int32_t split_len, void* out,
+                      void* workspace, int64_t workspace_bytes, int32_t* err, void* stream) {
   clear_error();
   MKV_REQUIRE(batch >= 0 && kv_units >= 0 && num_kv_heads > 0 && num_q_heads > 0 &&
                   max_seqlen_q >= 0 && num_q_tokens >= 0 && table_width >= 0 &&
                   table_stride >= table_width,
-              MKV_E_INVALID, "mkv_prefill_attention_bf16: bad sizes");
+              MKV_E_INVALID, "%s: bad sizes", fn);
   MKV_REQUIRE(head_dim == kPD, MKV_E_UNSUPPORTED,
-              "mkv_prefill_attention_bf16: head_dim %d unsupported (256)", head_dim);
+              "%s: head_dim %d unsupported (256)", fn,
+              head_dim);
   MKV_REQUIRE(num_q_heads == kPG * num_kv_heads, MKV_E_UNSUPPORTED,
-              "mkv_prefill_attention_bf16: %d query heads per KV head unsupported (4)",
+              "%s: %d query heads per KV head unsupported (4)", fn,
               num_q_heads / num_kv_heads);
   MKV_REQUIRE(num_q_heads <= 65535 && batch <= 65535, MKV_E_UNSUPPORTED,
-              "mkv_prefill_attention_bf16: batch or query heads above 65535");
-  MKV_REQUIRE(splits >= 1 && (splits == 1 || (split_len > 0 && split_len % kKvTile == 0)) &&
+              "%s: batch or query heads above 65535", fn);
+  MKV_REQUIRE(splits >= 1 &&
+                  (splits == 1 || planned || (split_len > 0 && split_len % kKvTile == 0)) &&
                   (int64_t)num_kv_heads * splits <= 65535,
-              MKV_E_INVALID, "mkv_prefill_attention_bf16: bad key split (%d x %d)", splits,
-              split_len);
+              MKV_E_INVALID, "%s: bad key split (%d x %d)", fn, splits, split_len);
   if (batch == 0 || max_seqlen_q == 0) return MKV_OK;
-  const int64_t need = mkv_prefill_attention_workspace_bytes(num_q_tokens, num_q_heads, splits);
-  MKV_REQUIRE(splits == 1 || (workspace && workspace_bytes >= need && aligned16(workspace)),
+  const int64_t part = mkv_prefill_attention_workspace_bytes(num_q_tokens, num_q_heads, splits);
+  const PlanSizes plan = plan_sizes(num_q_tokens, num_kv_heads, batch, max_seqlen_q, splits, kCus);
+  MKV_REQUIRE(!planned || (plan.tiles * num_kv_heads <= kPlanTiles && batch <= kPlanSeqs),
+              MKV_E_UNSUPPORTED, "%s: %lld query tiles or %d sequences unsupported (%d, %d)", fn,
+              (long long)plan.tiles * num_kv_heads, batch, kPlanTiles, kPlanSeqs);
+  const int64_t need = planned ? align16(part) + plan.bytes : part;
+  MKV_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned16(workspace)),
               MKV_E_INVALID,
-              "mkv_prefill_attention_bf16: workspace of %lld bytes (16-byte aligned) required",
-              (long long)need);
+              "%s: workspace of %lld bytes (16-byte aligned) required", fn, (long long)need);
   MKV_REQUIRE(q && k && v && cu_seqlens_q && out && err &&
                   (page_table ? seq_lens_k != nullptr : cu_seqlens_k != nullptr),
-              MKV_E_INVALID, "mkv_prefill_attention_bf16: null pointer");
+              MKV_E_INVALID, "%s: null pointer", fn);
   MKV_REQUIRE(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out), MKV_E_ALIGN,
-              "mkv_prefill_attention_bf16: q, k, v and out must be 16-byte aligned");
+              "%s: q, k, v and out must be 16-byte aligned", fn);
   PrefillArgs a;
   a.q = static_cast<const uint8_t*>(q);
   a.k = static_cast<const uint8_t*>(k);
@@ -643,9 +1006,13 @@ extern "C" int mkv_prefill_attention_bf16(const void* q, const void* k, const vo
   a.hkv = num_kv_heads;
   a.causal = causal ? 1 : 0;
   a.splits = splits;
-  a.split_len = splits > 1 ? split_len : 0;
+  a.split_len = splits > 1 && !planned ? split_len : INT_MAX / kKvTile * kKvTile;
   a.part = static_cast<float*>(workspace);
   a.ml = splits > 1 ? a.part + num_q_tokens * num_q_heads * splits * kPD : nullptr;
+  a.plan = nullptr;
+  a.items = a.cut = nullptr;
+  a.max_items = (int32_t)plan.items;
+  a.max_cuts = (int32_t)plan.cuts;
   // the kernel scales the row maximum, so its scale is positive: a negative
   // one flips the queries' signs, zero becomes the smallest normal number (the
   // masked scores stay -infinity under it)
@@ -653,22 +1020,93 @@ extern "C" int mkv_prefill_attention_bf16(const void* q, const void* k, const vo
   if (a.scale_log2 < FLT_MIN) a.scale_log2 = FLT_MIN;
   a.q_sign = softmax_scale < 0.f ? 0x80008000u : 0u;
   a.err = err;
+  const hipStream_t st = as_stream(stream);
+  a.rank0 = 0;
+  if (planned) {
+    a.plan = reinterpret_cast<Plan*>(static_cast<uint8_t*>(workspace) + align16(part));
+    a.items = reinterpret_cast<PlanItem*>(a.plan + 1);
+    a.cut = a.items + plan.items;
+    a.tok = kQTok;
+    a.ranks = 0;
+    if (batch <= kPlanSmall && plan.tiles <= kPlanSmall * kPlanSlots)
+      hipLaunchKernelGGL(prefill_plan_kernel<kPlanSmall>, dim3(1), dim3(kPlanSmall), 0, st, a, batch);
+    else
+      hipLaunchKernelGGL(prefill_plan_kernel<kPlanThreads>, dim3(1), dim3(kPlanThreads), 0, st, a,
+                         batch);
+    if (plan.items > 0)
+      hipLaunchKernelGGL(prefill_attn_kernel<8>, dim3((unsigned)plan.items), dim3(512), 0, st, a);
+    if (plan.cuts > 0)
+      hipLaunchKernelGGL(prefill_merge_kernel, dim3(kQTok, (unsigned)plan.cuts), dim3(256), 0, st,
+                         a);
+    return check_launch(fn);
+  }
   // Workgroups of 4 waves (32 query tokens) while they all fit the CUs at once:
   // each SIMD then has one wave to serve, so a key tile takes about half as
   // long. Past that, 8 waves share a tile's loads and overlap one another's
   // softmax with matrix work.
-  auto tiles = [&](int tok) {
-    return dim3((unsigned)((max_seqlen_q + (int64_t)tok - 1) / tok), (unsigned)batch,
-                (unsigned)(num_kv_heads * splits));
-  };
-  const dim3 small = tiles(kQTok / 2);
-  if ((int64_t)small.x * small.y * small.z <= kCus)
-    hipLaunchKernelGGL(prefill_attn_kernel<4>, small, dim3(256), 0, as_stream(stream), a);
-  else
-    hipLaunchKernelGGL(prefill_attn_kernel<8>, tiles(kQTok), dim3(512), 0, as_stream(stream), a);
+  const int64_t triples = (int64_t)batch * num_kv_heads * splits;
+  auto ranks = [&](int tok) { return (max_seqlen_q + (int64_t)tok - 1) / tok; };
+  const bool small = ranks(kQTok / 2) * triples <= kCus;
+  a.tok = small ? kQTok / 2 : kQTok;
+  a.ranks = (uint32_t)ranks(a.tok);
+  constexpr uint32_t kMaxZ = 65535;
+  for (a.rank0 = 0; a.rank0 < a.ranks; a.rank0 += kMaxZ) {
+    const dim3 grid((unsigned)(num_kv_heads * splits), (unsigned)batch,
+                    a.ranks - a.rank0 < kMaxZ ? a.ranks - a.rank0 : kMaxZ);
+    if (small)
+      hipLaunchKernelGGL(prefill_attn_kernel<4>, grid, dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL(prefill_attn_kernel<8>, grid, dim3(512), 0, st, a);
+  }
   if (splits > 1 && num_q_tokens > 0)
     hipLaunchKernelGGL(prefill_merge_kernel,
                        dim3((unsigned)max_seqlen_q, (unsigned)batch, (unsigned)num_kv_heads),
-                       dim3(256), 0, as_stream(stream), a);
-  return check_launch("mkv_prefill_attention_bf16");
+                       dim3(256), 0, st, a);
+  return check_launch(fn);
+}
+
+}  // namespace
+
+extern "C" int mkv_prefill_attention_bf16(const void* q, const void* k, const void* v,
+                                          int64_t kv_units, int32_t num_kv_heads,
+                                          int32_t num_q_heads, int32_t head_dim,
+                                          const int32_t* page_table, int64_t table_stride,
+                                          int32_t table_width, const int32_t* cu_seqlens_q,
+                                          const int32_t* cu_seqlens_k, const int32_t* seq_lens_k,
+                                          int32_t batch, int64_t num_q_tokens, int32_t max_seqlen_q,
+                                          float softmax_scale, int32_t causal, int32_t splits,
+                                          int32_t split_len, void* out, void* workspace,
+                                          int64_t workspace_bytes, int32_t* err, void* stream) {
+  return prefill_attention("mkv_prefill_attention_bf16", false, q, k, v, kv_units, num_kv_heads,
+                           num_q_heads, head_dim, page_table, table_stride, table_width,
+                           cu_seqlens_q, cu_seqlens_k, seq_lens_k, batch, num_q_tokens,
+                           max_seqlen_q, softmax_scale, causal, splits, split_len, out, workspace,
+                           workspace_bytes, err, stream);
+}
+
+extern "C" int mkv_prefill_attention_planned_bf16(
+    const void* q, const void* k, const void* v, int64_t kv_units, int32_t num_kv_heads,
+    int32_t num_q_heads, int32_t head_dim, const int32_t* page_table, int64_t table_stride,
+    int32_t table_width, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+    const int32_t* seq_lens_k, int32_t batch, int64_t num_q_tokens, int32_t max_seqlen_q,
+    float softmax_scale, int32_t causal, int32_t splits, void* out, void* workspace,
+    int64_t workspace_bytes, int32_t* err, void* stream) {
+  return prefill_attention("mkv_prefill_attention_planned_bf16", true, q, k, v, kv_units,
+                           num_kv_heads, num_q_heads, head_dim, page_table, table_stride,
+                           table_width, cu_seqlens_q, cu_seqlens_k, seq_lens_k, batch,
+                           num_q_tokens, max_seqlen_q, softmax_scale, causal, splits, 0, out,
+                           workspace, workspace_bytes, err, stream);
+}
+
+extern "C" int64_t mkv_prefill_attention_plan_bytes(int64_t num_q_tokens, int32_t num_q_heads,
+                                                    int32_t num_kv_heads, int32_t batch,
+                                                    int32_t max_seqlen_q, int32_t splits) {
+  if (num_q_tokens < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || batch < 0 ||
+      max_seqlen_q < 0 || splits <= 0)
+    return -1;
+  const PlanSizes s =
+      plan_sizes(num_q_tokens, num_kv_heads, batch, max_seqlen_q, splits, kCus);
+  if (s.tiles * num_kv_heads > kPlanTiles || batch > kPlanSeqs) return -1;
+  return align16(mkv_prefill_attention_workspace_bytes(num_q_tokens, num_q_heads, splits)) +
+         s.bytes;
 }

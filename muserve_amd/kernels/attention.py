@@ -15,6 +15,8 @@ word that ``check_errors(device)`` raises.
 """
 from __future__ import annotations
 
+import math
+
 import torch
 
 from muserve_amd import _lib
@@ -100,22 +102,53 @@ def attn_prefill_paged(
 PREFILL_Q_TILE = 64            # query tokens per workgroup of the prefill kernel
 PREFILL_KV_TILE = 64           # keys per step of the prefill kernel (key ranges are multiples)
 PREFILL_SPLIT_MIN = 256        # keys per range at least
+PREFILL_DENSE_MAX = 6          # key tiles per range up to which a launch is not planned
+PREFILL_PLAN_SEQS = 1024       # sequences, and query tiles x KV heads, of a planned launch
+PREFILL_PLAN_TILES = 4096
 _prefill_ws: dict[torch.device, torch.Tensor] = {}
-_prefill_min_wg: dict[torch.device, int] = {}
+_prefill_cu: dict[torch.device, int] = {}
 
 
-def _prefill_min_workgroups(dev: torch.device) -> int:
-    """Below this many query tiles, key ranges are split: one workgroup per
-    CU (the kernel's LDS allows one per CU). Measured on MI355X (256 CUs) in
-    the serving step, where the prefill attention runs beside the decode
-    attention: 256 gave 1.88 ms per step, 320 1.92, 384 1.91, 768 2.00 and
-    128 2.17 (more splits leave the decode attention fewer free CUs and
-    cost merge traffic; fewer leave CUs idle)."""
-    n = _prefill_min_wg.get(dev)
+def _prefill_cus(dev: torch.device) -> int:
+    n = _prefill_cu.get(dev)
     if n is None:
         n = torch.cuda.get_device_properties(dev).multi_processor_count
-        _prefill_min_wg[dev] = n
+        _prefill_cu[dev] = n
     return n
+
+
+def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: int, causal: bool,
+                     cus: int) -> tuple[int, int, bool]:
+    """(key ranges per query tile at most, keys a range aims at, planned).
+
+    A CU runs one workgroup at a time, a key tile after the other, so a launch
+    takes as long as the most key tiles that any CU gets. A grid sized on the
+    host (every query tile that the longest sequence could have, times the
+    batch, in ranges of the same number of keys) does while it fits the CUs at
+    once with short ranges; a planned launch sorts the tasks that exist on the
+    device, which costs a launch of 7-8 us and pays for itself where that
+    grid's ranges would be long or its sequences differ (MI355X: six prompts
+    of 80 to 4096 tokens 177 -> 143 us; 8 equal prompts of 4096, where the
+    grid is balanced as it is, take 254-262 us without a plan).
+    """
+    units = -(-max_k // PREFILL_KV_TILE)
+    rows = -(-max_q // PREFILL_Q_TILE)
+    dense = rows * batch
+    tiles = min(dense, tokens // PREFILL_Q_TILE + batch)
+    least = PREFILL_SPLIT_MIN // PREFILL_KV_TILE
+    fit = cus // max(1, dense * kv_heads)
+    aim = max(least, -(-units // fit)) if fit else units
+    if units <= least or aim <= PREFILL_DENSE_MAX:
+        splits = max(1, -(-units // aim)) if fit else 1
+        return (splits, aim * PREFILL_KV_TILE, False) if splits > 1 else (1, 0, False)
+    mean = units - (min(rows, units) - 1) / 2 if causal else units
+    share = tiles * kv_heads * mean / cus  # key tiles per CU, at most
+    if batch > PREFILL_PLAN_SEQS or tiles * kv_heads > PREFILL_PLAN_TILES:
+        return 1, 0, False
+    if share >= units:  # several rounds of whole tiles: long enough to balance by their order
+        return 1, 0, dense > tiles + tiles // 8
+    splits = -(-units // max(least, int(share * 3 / 4)))
+    return min(splits, 65535 // kv_heads), 0, True
 
 
 def _prefill(q, k, v, page_table, cu_q, cu_k, lens_k, max_seqlen_q, softmax_scale, causal, out,
@@ -152,31 +185,29 @@ def _prefill(q, k, v, page_table, cu_q, cu_k, lens_k, max_seqlen_q, softmax_scal
         raise ValueError("out must be a contiguous tensor shaped like q")
     scale = D ** -0.5 if softmax_scale is None else float(softmax_scale)
     units = k.shape[0]
-    # key-range splits when the query tiles alone would leave most CUs idle
     max_k = int(max_seqlen_k) if max_seqlen_k is not None else page_table.shape[1] * 16
-    tiles = -(-int(max_seqlen_q) // PREFILL_Q_TILE) * batch * Hkv
-    splits = 1
-    min_wg = _prefill_min_workgroups(dev)
-    if tiles < min_wg and max_k > PREFILL_SPLIT_MIN:
-        splits = min(-(-min_wg // max(tiles, 1)), -(-max_k // PREFILL_SPLIT_MIN))
-    split_len = -(-max_k // splits // PREFILL_KV_TILE) * PREFILL_KV_TILE if splits > 1 else 0
-    if splits > 1:
-        splits = -(-max_k // split_len)
+    splits, split_len, planned = prefill_schedule(Tq, int(max_seqlen_q), max_k, batch, Hkv, causal,
+                                                  _prefill_cus(dev))
     ws, ws_bytes = None, 0
-    if splits > 1:
+    if planned:
+        ws_bytes = _lib.load().mkv_prefill_attention_plan_bytes(Tq, Hq, Hkv, batch,
+                                                                int(max_seqlen_q), splits)
+    elif splits > 1:
         ws_bytes = _lib.load().mkv_prefill_attention_workspace_bytes(Tq, Hq, splits)
+    if ws_bytes > 0:
         ws = _prefill_ws.get(dev)
         if ws is None or ws.numel() < ws_bytes:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
             _prefill_ws[dev] = ws
     # the workspace is reused by later calls on the stream: calls on one
     # device must be issued on one stream (or be ordered by the caller)
-    _lib.call("mkv_prefill_attention_bf16", q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv,
+    fn = "mkv_prefill_attention_planned_bf16" if planned else "mkv_prefill_attention_bf16"
+    _lib.call(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv,
               Hq, D, _lib.ptr(page_table), page_table.stride(0) if page_table is not None else 0,
               page_table.shape[1] if page_table is not None else 0, cu_q.data_ptr(),
               _lib.ptr(cu_k), _lib.ptr(lens_k), batch, Tq, int(max_seqlen_q), scale,
-              1 if causal else 0, splits, split_len, out.data_ptr(), _lib.ptr(ws), ws_bytes,
-              _errword(dev).ptr(), _lib.stream_of(dev))
+              1 if causal else 0, splits, *(() if planned else (split_len,)), out.data_ptr(),
+              _lib.ptr(ws), ws_bytes, _errword(dev).ptr(), _lib.stream_of(dev))
     return out
 
 

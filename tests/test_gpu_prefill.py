@@ -353,3 +353,60 @@ def test_query_tiles_scales_and_rising_maxima(lens, scale, grow):
     want = att.prefill_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(),
                                  cu.numpy(), scale, True, cu_k=cu.numpy(), stats=True)
     within(out, want)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("splits,heads,nqs,nks", [
+    # both sides of the 64-query and 64-key tiles, no queries, no visible keys
+    (1, 1, [1, 0, 63, 64, 65, 129, 70], [1, 9, 64, 127, 65, 300, 20]),
+    (2, 2, [1, 65, 0, 64, 200], [777, 65, 0, 640, 200]),
+    (16, 1, [130, 1, 700, 64], [1500, 2049, 700, 64]),   # all tasks at once: ranges of 2 tiles up
+    (40, 1, [20], [2560]),                               # many ranges of one query tile
+    (3, 1, [1900, 1200] + [64] * 220, [1900, 1200] + [64] * 220),  # more tasks than CUs
+    (5, 4, [300] * 30, [960] * 30),                      # 600 tasks of one length over 4 heads
+])
+def test_planned_launches_pin_every_task(splits, heads, nqs, nks, causal):
+    """The schedule made on the device: with zero queries over one-hot keys a
+    task dropped, doubled or cut in the wrong place changes what a row counts.
+    Output rows past the queries stay as they were."""
+    case(f"prefill planned: {len(nqs)} sequences, {heads} heads, {splits} ranges, causal={causal}")
+    Tq, Tk = sum(nqs), sum(nks)
+    cu_q = torch.tensor(np.cumsum([0] + nqs), dtype=torch.int32, device=DEV)
+    cu_k = torch.tensor(np.cumsum([0] + nks), dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(43)
+    q = torch.zeros(Tq, 4 * heads, 256).bfloat16().to(DEV)
+    k = torch.randn(Tk, heads, 256, generator=g).bfloat16().to(DEV)
+    v = torch.cat([_one_hot_keys(n, heads) for n in nks]).to(DEV)
+    out = torch.full((Tq + 8, 4 * heads, 256), 7.0, dtype=torch.bfloat16, device=DEV)
+    n = _lib.load().mkv_prefill_attention_plan_bytes(Tq, 4 * heads, heads, len(nqs), max(nqs),
+                                                     splits)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    _lib.call("mkv_prefill_attention_planned_bf16", q.data_ptr(), k.data_ptr(), v.data_ptr(), Tk,
+              heads, 4 * heads, 256, None, 0, 0, cu_q.data_ptr(), cu_k.data_ptr(), None, len(nqs),
+              Tq, max(nqs), 256 ** -0.5, int(causal), splits, out.data_ptr(), ws.data_ptr(), n,
+              A._errword(DEV).ptr(), _lib.stream_of(DEV))
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    off = 0
+    for nq, nk in zip(nqs, nks):
+        want = _one_hot_want(nq, nk, causal)
+        for h in range(4 * heads):
+            if nq:
+                _bf16_close(out[off:off + nq, h], want)
+        off += nq
+    assert bool((out[Tq:] == 7.0).all())
+
+
+@pytest.mark.parametrize("tokens,max_q,max_k,batch,heads", [
+    (1, 1, 1, 1, 1), (77, 77, 77, 1, 1), (13897, 4096, 4096, 6, 1), (32768, 4096, 4096, 8, 1),
+    (2572, 1428, 6540, 2, 1), (3, 1, 1 << 20, 3, 2), (4096, 16, 64, 256, 1),
+    (1 << 20, 1 << 20, 1 << 20, 1, 1), (5000, 4096, 4096, 1100, 1), (200, 200, 9000, 1, 8)])
+def test_schedules_are_accepted(tokens, max_q, max_k, batch, heads):
+    """Every schedule the host rule makes is one the entry points take."""
+    splits, split_len, planned = A.prefill_schedule(tokens, max_q, max_k, batch, heads, True, 256)
+    assert splits >= 1 and heads * splits <= 65535
+    if planned:
+        assert _lib.load().mkv_prefill_attention_plan_bytes(tokens, 4 * heads, heads, batch, max_q,
+                                                            splits) > 0
+    elif splits > 1:
+        assert split_len > 0 and split_len % 64 == 0 and splits * split_len >= max_k

@@ -897,6 +897,10 @@ __global__ __launch_bounds__(kAttnThreads, G == 8 ? 1 : 2) void attn_span_kernel
 // wave index not uniform) made the prefix-reuse serving step 1.7-2.6 %
 // slower while their merges were faster.
 constexpr int kMergeBatch = 4;   // pieces a wave loads at once (more pieces)
+// With fewer pairs than this the launch's waves leave more than kMergeExact
+// pieces a pair on average, and nothing fills the GPU beside a merge of so few
+// workgroups: the wide form.
+constexpr int kMergeWidePairs = 128;
 constexpr int kMergeExact = 16;  // pieces merged by one thread per dim in one batch
 
 // The merge of a pair with exactly N pieces, a thread per dim: every load is
@@ -925,10 +929,15 @@ __device__ __forceinline__ float merge_exact(const AttnArgs& a, AtOf at_of, int 
   return L > 0.f ? O / L : 0.f;
 }
 
-template <int G, bool F16>
-__global__ __launch_bounds__(kAttnThreads) void attn_merge_kernel(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) float wave_o[kAttnWaves][kHeadDim];
-  __shared__ float wave_ml[kAttnWaves][2];
+// WAVES 4, BATCH 4: the form above, 16 pieces a round trip. WAVES 16, BATCH 8:
+// for few pairs, whose pieces are many (the grid's waves over the pairs): 128
+// pieces a round trip. 17 sequences x 2 KV heads, at most 194 pieces a pair:
+// 11.9 -> 5.3 us, the whole decode step 31.6 -> 25.3 us; one sequence of 49
+// pieces: 4.6 -> 4.0 us.
+template <int G, bool F16, int WAVES, int BATCH>
+__global__ __launch_bounds__(64 * WAVES) void attn_merge_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) float wave_o[WAVES][kHeadDim];
+  __shared__ float wave_ml[WAVES][2];
   const int64_t pr = blockIdx.x / G;
   const int h = blockIdx.x % G;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -940,7 +949,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_merge_kernel(AttnArgs a) {
   asm volatile("" ::"s"(span));
   uint8_t* out = a.out + (pr * G + h) * kRowBytes;
   if (p1 <= p0) {  // nothing to attend to: zeros
-    reinterpret_cast<uint16_t*>(out)[tid] = 0;
+    if (tid < kHeadDim) reinterpret_cast<uint16_t*>(out)[tid] = 0;
     return;
   }
   // flat page indices are int32, and the span is at most the launch's pages
@@ -956,6 +965,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_merge_kernel(AttnArgs a) {
     return (w * 2 + slot) * G + h;
   };
   if (n_seg <= kMergeExact) {  // most cut pairs: one round trip, no duplicate loads
+    if (tid >= kHeadDim) return;  // whole waves
     float r;
     switch (n_seg) {
       case 2: r = merge_exact<2>(a, at_of, tid); break;
@@ -979,34 +989,34 @@ __global__ __launch_bounds__(kAttnThreads) void attn_merge_kernel(AttnArgs a) {
   }
   float m_run = -INFINITY, l_run = 0.f;
   f32x4 o_run = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int i0 = wave; i0 < n_seg; i0 += kAttnWaves * kMergeBatch) {
-    const int mine = i0 + kAttnWaves * (lane & (kMergeBatch - 1));
+  for (int i0 = wave; i0 < n_seg; i0 += WAVES * BATCH) {
+    const int mine = i0 + WAVES * (lane & (BATCH - 1));
     const float2 ml =
         *reinterpret_cast<const float2*>(a.ml + at_of(mine < n_seg ? mine : n_seg - 1) * 2);
-    f32x4 p[kMergeBatch];
+    f32x4 p[BATCH];
 #pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      const int i = i0 + kAttnWaves * u;
+    for (int u = 0; u < BATCH; ++u) {
+      const int i = i0 + WAVES * u;
       p[u] = *reinterpret_cast<const f32x4*>(a.part + at_of(i < n_seg ? i : n_seg - 1) * kHeadDim +
                                              4 * lane);
     }
-    float m[kMergeBatch], l[kMergeBatch];
+    float m[BATCH], l[BATCH];
 #pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
+    for (int u = 0; u < BATCH; ++u) {
       m[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ml.x), u));
       l[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ml.y), u));
     }
     float mb = m_run;
 #pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u)
-      mb = fmaxf(mb, i0 + kAttnWaves * u < n_seg ? m[u] : -INFINITY);
+    for (int u = 0; u < BATCH; ++u)
+      mb = fmaxf(mb, i0 + WAVES * u < n_seg ? m[u] : -INFINITY);
     // mb >= m_run; a wave's first batch starts from nothing
     const float alpha = m_run == -INFINITY ? 0.f : exp2_fast(m_run - mb);
     l_run *= alpha;
     o_run *= alpha;
 #pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      const bool ok = i0 + kAttnWaves * u < n_seg;
+    for (int u = 0; u < BATCH; ++u) {
+      const bool ok = i0 + WAVES * u < n_seg;
       const float f = !ok || m[u] == -INFINITY ? 0.f : exp2_fast(m[u] - mb);
 #pragma unroll
       for (int e = 0; e < 4; ++e) o_run[e] += f * (ok ? p[u][e] : -0.f);
@@ -1020,12 +1030,13 @@ __global__ __launch_bounds__(kAttnThreads) void attn_merge_kernel(AttnArgs a) {
     wave_ml[wave][1] = l_run;
   }
   __syncthreads();
+  if (tid >= kHeadDim) return;
   float M = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < kAttnWaves; ++w) M = fmaxf(M, wave_ml[w][0]);
+  for (int w = 0; w < WAVES; ++w) M = fmaxf(M, wave_ml[w][0]);
   float O = 0.f, L = 0.f;
 #pragma unroll
-  for (int w = 0; w < kAttnWaves; ++w) {
+  for (int w = 0; w < WAVES; ++w) {
     const float mw = wave_ml[w][0];
     const float f = mw == -INFINITY ? 0.f : exp2_fast(mw - M);
     O += f * wave_o[w][tid];
@@ -1112,8 +1123,12 @@ int launch_attn(AttnArgs a, int grid, hipStream_t st) {
   else
     hipLaunchKernelGGL((attn_span_kernel<G, FP8, F16, false>), dim3((unsigned)grid),
                        dim3(kAttnThreads), lds, st, a);
-  hipLaunchKernelGGL((attn_merge_kernel<G, F16>), dim3((unsigned)(a.pairs * G)),
-                     dim3(kAttnThreads), 0, st, a);
+  if (a.pairs < kMergeWidePairs)
+    hipLaunchKernelGGL((attn_merge_kernel<G, F16, 16, 8>), dim3((unsigned)(a.pairs * G)),
+                       dim3(16 * 64), 0, st, a);
+  else
+    hipLaunchKernelGGL((attn_merge_kernel<G, F16, kAttnWaves, kMergeBatch>),
+                       dim3((unsigned)(a.pairs * G)), dim3(kAttnThreads), 0, st, a);
   return MKV_OK;
 }
 

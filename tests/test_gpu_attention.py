@@ -84,6 +84,20 @@ def test_matches_oracle(Hq, Hkv):
     within_one_ulp(got, want)
 
 
+@pytest.mark.parametrize("lens", [
+    [16 * 16], [16 * 17], [16 * 127 + 5], [16 * 128], [16 * 129],  # pieces of one page each
+    [16 * 1200 + 1, 0, 9], [16 * 2049],                            # many a wave of the merge
+    [20] * 126 + [16 * 300], [20] * 127 + [16 * 300],              # pairs around the wide merge's
+])
+def test_merge_of_few_pairs(lens):
+    """Both forms of the merge around the piece counts where a pair goes from
+    one batch to several, and around the pair count that chooses the form."""
+    case(f"decode attention merge: {len(lens)} sequences, longest {max(lens)}")
+    q, k, v, lens, table = build(31 + len(lens), lens, 4, 1)
+    got, want = run(q, k, v, lens, table)
+    within_one_ulp(got, want)
+
+
 def test_tight_bound_and_scale():
     lens = [300, 64, 511, 1]
     case(f"decode attention, max_seqlen 512 (no merge pass), scale 0.1, lens {lens}")

@@ -38,3 +38,14 @@ def test_page_hashes_workgroup_without_pages():
     assert cu_p[32] == 0
     for r, x in enumerate(ids):
         assert got[cu_p[r]:cu_p[r + 1]].tolist() == ref.page_hashes(x), r
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.int32])
+@pytest.mark.parametrize("pages", [0, 1, 2, 3, 4, 5])
+def test_page_hashes_of_one_request(pages, dtype):
+    """Odd and even step counts of a workgroup: its steps run in pairs, each
+    holding the next one's schedule."""
+    case(f"page hashes of one request of {pages} pages, {np.dtype(dtype).name}")
+    x = np.random.default_rng(pages).integers(0, 151936, 16 * pages + 7).astype(dtype)
+    h, _ = page_hashes(torch.from_numpy(x).to(DEV), np.array([0, len(x)]))
+    assert as_u64(h)[:pages].tolist() == ref.page_hashes(x)

@@ -41,7 +41,7 @@ def test_page_hashes_workgroup_without_pages():
 
 
 @pytest.mark.parametrize("dtype", [np.int64, np.int32])
-@pytest.mark.parametrize("pages", [0, 1, 2, 3, 4, 5])
+@pytest.mark.parametrize("pages", [1, 2, 3, 4, 5])
 def test_page_hashes_of_one_request(pages, dtype):
     """Odd and even step counts of a workgroup: its steps run in pairs, each
     holding the next one's schedule."""

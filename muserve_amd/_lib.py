@@ -177,7 +177,7 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 f"muserve_amd kernels run on a ROCm GPU only; got a tensor on {t.device}")
         if dev is None:

@@ -23,6 +23,9 @@ from muserve_amd import _lib
 
 HEAD_DIM = 256
 
+_DECODE_FNS = {torch.bfloat16: "mkv_decode_attention_bf16",
+               torch.float16: "mkv_decode_attention_f16"}
+
 _errors: dict[torch.device, _lib.DeviceErrors] = {}
 _workspace: dict[torch.device, torch.Tensor] = {}
 
@@ -240,12 +243,11 @@ def attn_decode(
     ``cache_seqlens[b]`` rows attended (the reference forwards None to its
     kernel the same way, muserve/kernels/attention.py:33-42): the padded
     layout ``PagedKVCache.gather`` writes."""
-    fns = {torch.bfloat16: "mkv_decode_attention_bf16", torch.float16: "mkv_decode_attention_f16"}
-    if k_cache.dtype not in fns or v_cache.dtype != k_cache.dtype:
+    if k_cache.dtype not in _DECODE_FNS or v_cache.dtype != k_cache.dtype:
         raise TypeError("attn_decode takes bf16 or fp16 caches (attn_decode_fp8 reads fp8 ones)")
     if q.dtype != k_cache.dtype:
         raise TypeError(f"q is {q.dtype}, the caches {k_cache.dtype}: they must match")
-    return _decode(fns[k_cache.dtype], q, k_cache, v_cache, None, None, cache_seqlens,
+    return _decode(_DECODE_FNS[k_cache.dtype], q, k_cache, v_cache, None, None, cache_seqlens,
                    page_table, softmax_scale, max_seqlen, out, shared_pages)
 
 

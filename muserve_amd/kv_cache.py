@@ -229,13 +229,17 @@ class PagedKVCache:
             if not (-self.num_layers <= first < self.num_layers):
                 raise IndexError(f"layer {layer} out of range for {self.num_layers} layers")
             first %= self.num_layers
-            k, v = k.unsqueeze(0), v.unsqueeze(0)
-        want = (L, T, self.kv_heads, self.head_dim)
-        if tuple(k.shape) != want or tuple(v.shape) != want:
+        rows = (T, self.kv_heads, self.head_dim)
+        want = (L, *rows) if layer is None else rows
+        if k.shape != want or v.shape != want:
             raise ValueError(f"k/v must be {want}, got {tuple(k.shape)} / {tuple(v.shape)}")
+        # conversions are no-ops in a decode step, whose host time is a dozen
+        # such calls: they are made only where something differs
         in_dtype = torch.bfloat16 if self.dtype == _FP8 else self.dtype
-        k = k.to(device=dev, dtype=in_dtype).contiguous()
-        v = v.to(device=dev, dtype=in_dtype).contiguous()
+        if k.dtype != in_dtype or k.device != dev or not k.is_contiguous():
+            k = k.to(device=dev, dtype=in_dtype).contiguous()
+        if v.dtype != in_dtype or v.device != dev or not v.is_contiguous():
+            v = v.to(device=dev, dtype=in_dtype).contiguous()
         _lib.require_gpu(k, v, slot_mapping, self.cache)
         if T == 0:
             return
@@ -243,20 +247,23 @@ class PagedKVCache:
             if self._unique is None:
                 self._unique = _lib.UniqueCheck(dev, self.num_slots)
             self._unique.run(slot_mapping, self._errors)
+        # the layer's planes by address (views of them are two indexings each)
         esz = self.cache.element_size()
-        kp = self.cache[first, 0]
-        vp = self.cache[first, 1]
+        plane = self.num_slots * self.row_elems * esz
+        kp = self.cache.data_ptr() + 2 * first * plane
+        vp = kp + plane
         src_layer = T * self.row_elems * 2
         src_tok = self.row_elems * 2
         stream = _lib.stream_of(dev)
         if self.dtype == _FP8:
-            _lib.call("mkv_append_fp8", kp.data_ptr(), vp.data_ptr(),
-                      self.scales[first, 0].data_ptr(), self.scales[first, 1].data_ptr(),
+            splane = self.num_slots * self.kv_heads * 4
+            ks = self.scales.data_ptr() + 2 * first * splane
+            _lib.call("mkv_append_fp8", kp, vp, ks, ks + splane,
                       self._plane_layer_stride(), self._scale_layer_stride(), self.num_slots,
                       k.data_ptr(), v.data_ptr(), src_layer, src_tok, slot_mapping.data_ptr(), T,
                       L, self.kv_heads, self.head_dim, self._errors.ptr(), stream)
         else:
-            _lib.call("mkv_append_bf16", kp.data_ptr(), vp.data_ptr(), self._plane_layer_stride(),
+            _lib.call("mkv_append_bf16", kp, vp, self._plane_layer_stride(),
                       self.num_slots, k.data_ptr(), v.data_ptr(), src_layer, src_tok,
                       slot_mapping.data_ptr(), T, L, self.row_elems * esz, self._errors.ptr(),
                       stream)
@@ -264,6 +271,9 @@ class PagedKVCache:
     def get_kv_by_layer(self, layer_idx: int):
         """(k_cache, v_cache) views [num_pages, 16, kv_heads, head_dim]
         (muserve/kv_cache.py:114-118), as flash_attn_with_kvcache reads them."""
+        if type(layer_idx) is int:  # two selects of one layer, not four indexings
+            layer = self.cache.select(0, layer_idx)
+            return layer.select(0, 0), layer.select(0, 1)
         return self.cache[layer_idx, 0], self.cache[layer_idx, 1]
 
     def gather(self, layer: int | None, block_tables: torch.Tensor, seq_lens: torch.Tensor,

@@ -125,27 +125,44 @@ __global__ __launch_bounds__(kHashThreads) void block_hash_kernel(const uint8_t*
 
   Sha256 st;  // rounds wave: the even lane's running state; the odd lane's to finalise
   sha256_init(st);
+  if (steps == 0) return;  // uniform: both waves hold the same requests
+  // Before the first rounds both waves make a schedule: the schedule wave step
+  // 0's, the rounds wave step 1's (no page is finished before step bpp, and
+  // step 1 finishes page 0 only where a page is one block).
+  {
+    const int64_t u = rounds ? 1 : 0;
+    uint32_t w[16];
+    if (!finisher && u < nblk) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) w[j] = bswap32(p[16 * u + j]);
+      sha256_kw_store(w, col_base + u * 16 * 64);
+    } else if (finisher && u == bpp && pages >= 1) {
+      sha256_pad_block(w, page_bytes);
+      sha256_kw_store(w, col_base + u * 16 * 64);
+    }
+  }
+  __syncthreads();
   // schedule wave: the even lane holds the next block's words
   uint32_t next[16];
 #pragma unroll
   for (int j = 0; j < 16; ++j) next[j] = 0;
-  if (!rounds && !finisher && nblk > 0) {
+  if (!rounds && !finisher && nblk > 2) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) next[j] = p[j];
+    for (int j = 0; j < 16; ++j) next[j] = p[32 + j];
   }
   // Iteration s: the rounds wave loads step s + 1's K + W (from buffer
   // (s + 1) & 1) and compresses step s from registers, while the schedule wave
   // fills step s + 2 (buffer s & 1, whose step the rounds wave holds since
-  // iteration s - 1); one barrier ends the iteration for both waves. Step u
+  // iteration s - 1, or from before the first); one barrier ends the iteration for both waves. Step u
   // is block u % bpp of page u / bpp. Two iterations are unrolled, so that
   // the two register sets swap by name.
   const int log_bpp = bpp - 1;
   auto iteration = [&](int64_t s, uint32_t (&now)[64], uint32_t (&after)[64])
                        __attribute__((always_inline)) {
     if (rounds) {
-      if (s >= -1) sha256_kw_load(after, col_base + ((s + 1) & 1) * 16 * 64);
+      sha256_kw_load(after, col_base + ((s + 1) & 1) * 16 * 64);
       __builtin_amdgcn_sched_barrier(0);
-      if (s >= 0 && s < steps) {
+      if (s < steps) {
         sha256_rounds_kw(st, now);
         const int64_t i = s >> log_bpp;
         const int k = (int)(s & log_bpp);
@@ -191,7 +208,9 @@ __global__ __launch_bounds__(kHashThreads) void block_hash_kernel(const uint8_t*
   uint32_t kw_a[64], kw_b[64];
 #pragma unroll
   for (int t = 0; t < 64; ++t) kw_a[t] = kw_b[t] = 0;
-  for (int64_t s = -2; s < steps; s += 2) {
+  if (rounds) sha256_kw_load(kw_a, col_base);
+  __syncthreads();
+  for (int64_t s = 0; s < steps; s += 2) {
     iteration(s, kw_a, kw_b);
     iteration(s + 1, kw_b, kw_a);
   }

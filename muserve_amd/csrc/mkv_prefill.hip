@@ -112,9 +112,10 @@ struct PrefillArgs {
   uint8_t* out;          // [Tq, Hq, 256] bf16
   int32_t hkv;
   int32_t causal;
-  int32_t tok;           // query tokens per workgroup of this launch
+  int32_t tok;           // query tokens per workgroup of this launch (a power of two)
   uint32_t ranks;        // query tiles of the longest sequence the launch covers
   uint32_t rank0;        // the first tile rank of this launch
+  int32_t turn;          // the grid is more than the CUs: ranks turn over the XCDs
   int32_t splits;        // key ranges per (query tile, KV head) at most
   int32_t split_len;     // keys a range aims at (a multiple of the KV tile)
   Plan* plan;            // null: the grid is the schedule
@@ -201,12 +202,13 @@ __device__ __forceinline__ int64_t tile_end(const PrefillArgs& a, int64_t nk, in
 }
 
 // Key ranges of a query tile that sees `units` key tiles: as many as keep a
-// range at `cap` key tiles, at most the launch's count. Range z of p covers
-// the key tiles from units * z / p to units * (z + 1) / p. A query tile of one
-// range is written by its workgroup, with no partial rows and no merge.
+// range at `cap` key tiles, at most the launch's count. The ranges differ by at
+// most one key tile, the longer ones first. A query tile of one range is
+// written by its workgroup, with no partial rows and no merge.
 __device__ __forceinline__ int32_t tile_ranges(int32_t units, int32_t cap, int32_t splits) {
-  const int32_t p = (units + cap - 1) / cap;
-  return p > splits ? splits : p < 1 ? 1 : p;
+  if (units <= cap) return 1;
+  const int32_t p = (int32_t)((uint32_t)(units + cap - 1) / (uint32_t)cap);
+  return p > splits ? splits : p;
 }
 __device__ __forceinline__ int32_t units_of(int64_t keys) {
   return (int32_t)((keys + kKvTile - 1) / kKvTile);
@@ -275,23 +277,31 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
     // head, range) triples of a rank before the next rank. The dispatcher
     // hands consecutive workgroups to the 8 XCDs in turn, whatever their
     // load, so a triple moves one XCD on with every 8 workgroups: each XCD
-    // gets tiles of all ranks of every sequence.
-    const uint32_t triples = gridDim.x * gridDim.y;
+    // gets tiles of all ranks of every sequence. (A grid no larger than the
+    // CUs runs at once, in any order: no turn, and no divisions for it.
+    // Without the turn, sequences of 79, 76, 731 and 916 tokens took 42 us.)
     const uint32_t rank = a.rank0 + blockIdx.z;
-    const uint64_t turn = triples >= kXcds ? rank : (uint64_t)rank * triples / kXcds;
-    uint32_t at = (uint32_t)(((uint64_t)blockIdx.y * gridDim.x + blockIdx.x + turn) % triples);
-    split = (int32_t)(at % (uint32_t)a.splits);
-    at /= (uint32_t)a.splits;
-    b = at / (uint32_t)a.hkv;
-    hk = at % (uint32_t)a.hkv;
-    bool bad;
-    nq = seq_queries(a, b, qs, bad);
-    if (bad && tid == 0 && rank == 0 && split == 0 && hk == 0) raise_err(a.err, MKV_DEVERR_TABLE);
+    uint32_t at = blockIdx.x;
+    b = blockIdx.y;
+    if (a.turn) {
+      const uint32_t triples = gridDim.x * gridDim.y;
+      const uint32_t turn =
+          triples >= kXcds ? rank % triples : (uint32_t)((uint64_t)rank * triples / kXcds) % triples;
+      uint64_t to = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x + turn;
+      to = to >= triples ? to - triples : to;
+      b = (uint32_t)to / gridDim.x;
+      at = (uint32_t)to - (uint32_t)b * gridDim.x;
+    }
+    hk = a.splits == 1 ? at : at / (uint32_t)a.splits;
+    split = (int32_t)(at - (uint32_t)hk * (uint32_t)a.splits);
+    bool bad_q, bad_k;
+    nq = seq_queries(a, b, qs, bad_q);
+    nk = seq_keys(a, b, kbase, bad_k);  // (its loads go out with the queries')
+    if (bad_q && tid == 0 && rank == 0 && split == 0 && hk == 0) raise_err(a.err, MKV_DEVERR_TABLE);
     const int64_t q = (int64_t)(a.ranks - 1 - rank) * kTok;  // the workgroup's first query
     if (q >= nq) return;  // uniform
     qt = (int32_t)q;
-    nk = seq_keys(a, b, kbase, bad);
-    if (bad && tid == 0 && qt == 0) raise_err(a.err, MKV_DEVERR_TABLE);
+    if (bad_k && tid == 0 && qt == 0) raise_err(a.err, MKV_DEVERR_TABLE);
     ranges = tile_ranges(units_of(tile_end(a, nk, nq, qt)), a.split_len / kKvTile, a.splits);
     if (split >= ranges) return;  // uniform
   }
@@ -303,9 +313,11 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
   // this workgroup's key range
   int64_t kv_end = tile_end(a, nk, nq, qt), kv_begin = 0;
   if (ranges > 1) {
-    const int64_t units = units_of(kv_end);
-    kv_begin = units * split / ranges * kKvTile;
-    if (split + 1 < ranges) kv_end = units * (split + 1) / ranges * kKvTile;
+    const uint32_t units = (uint32_t)units_of(kv_end);
+    const uint32_t each = units / (uint32_t)ranges, more = units - each * (uint32_t)ranges;
+    const uint32_t z = (uint32_t)split;
+    kv_begin = (int64_t)(z * each + (z < more ? z : more)) * kKvTile;
+    if (split + 1 < ranges) kv_end = kv_begin + (int64_t)(each + (z < more ? 1 : 0)) * kKvTile;
   }
   // the last key any of this wave's queries sees (-1: it has none), and the
   // last one that all of them see
@@ -649,12 +661,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     int64_t kbase;
     bool bad;
     const int32_t nq = seq_queries(a, b, qs, bad);
+    const int64_t nk = seq_keys(a, b, kbase, bad);
     t = blockIdx.x;
     hk = blockIdx.z;
     if (t >= nq) return;
-    const int64_t nk = seq_keys(a, b, kbase, bad);
-    ranges = tile_ranges(units_of(tile_end(a, nk, nq, t / a.tok * a.tok)),
-                         a.split_len / kKvTile, a.splits);
+    ranges = tile_ranges(units_of(tile_end(a, nk, nq, t & -a.tok)), a.split_len / kKvTile,
+                         a.splits);
     if (ranges == 1) return;
   }
   const int64_t row = ((int64_t)qs + t) * ((int64_t)a.hkv * kPG) +
@@ -1028,6 +1040,7 @@ int prefill_attention(const char* fn, bool planned, const void* q, const void* k
     a.cut = a.items + plan.items;
     a.tok = kQTok;
     a.ranks = 0;
+    a.turn = 0;
     if (batch <= kPlanSmall && plan.tiles <= kPlanSmall * kPlanSlots)
       hipLaunchKernelGGL(prefill_plan_kernel<kPlanSmall>, dim3(1), dim3(kPlanSmall), 0, st, a, batch);
     else
@@ -1040,15 +1053,19 @@ int prefill_attention(const char* fn, bool planned, const void* q, const void* k
                          a);
     return check_launch(fn);
   }
-  // Workgroups of 4 waves (32 query tokens) while they all fit the CUs at once:
-  // each SIMD then has one wave to serve, so a key tile takes about half as
-  // long. Past that, 8 waves share a tile's loads and overlap one another's
-  // softmax with matrix work.
-  const int64_t triples = (int64_t)batch * num_kv_heads * splits;
+  // Workgroups of 4 waves (32 query tokens) while the ones with work fit the CUs
+  // at once: each SIMD then has one wave to serve, so a key tile takes about
+  // half as long. Past that, 8 waves share a tile's loads and overlap one
+  // another's softmax with matrix work. The rows bound the tiles that exist
+  // (sequences of 79, 76, 731 and 916 tokens in 4 ranges: 464 workgroups of 4
+  // waves, at most 240 with work).
   auto ranks = [&](int tok) { return (max_seqlen_q + (int64_t)tok - 1) / tok; };
-  const bool small = ranks(kQTok / 2) * triples <= kCus;
+  const int64_t dense = ranks(kQTok / 2) * batch, rows = num_q_tokens / (kQTok / 2) + batch;
+  const bool small = (dense < rows ? dense : rows) * num_kv_heads * splits <= kCus;
+  const int64_t triples = (int64_t)batch * num_kv_heads * splits;
   a.tok = small ? kQTok / 2 : kQTok;
   a.ranks = (uint32_t)ranks(a.tok);
+  a.turn = (int64_t)a.ranks * triples > kCus;
   constexpr uint32_t kMaxZ = 65535;
   for (a.rank0 = 0; a.rank0 < a.ranks; a.rank0 += kMaxZ) {
     const dim3 grid((unsigned)(num_kv_heads * splits), (unsigned)batch,

@@ -143,7 +143,8 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     aim = max(least, -(-units // fit)) if fit else units
     if units <= least or aim <= PREFILL_DENSE_MAX:
         splits = max(1, -(-units // aim)) if fit else 1
-        return (splits, aim * PREFILL_KV_TILE, False) if splits > 1 else (1, 0, False)
+        per = -(-units // splits)
+        return (splits, per * PREFILL_KV_TILE, False) if splits > 1 else (1, 0, False)
     mean = units - (min(rows, units) - 1) / 2 if causal else units
     share = tiles * kv_heads * mean / cus  # key tiles per CU, at most
     if batch > PREFILL_PLAN_SEQS or tiles * kv_heads > PREFILL_PLAN_TILES:

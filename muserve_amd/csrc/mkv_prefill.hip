@@ -684,16 +684,36 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     case 6: merge_ranges<6>(ml, part, L, O); break;
     case 7: merge_ranges<7>(ml, part, L, O); break;
     case 8: merge_ranges<8>(ml, part, L, O); break;
-    default: {  // more than 8 ranges
+    default: {
+      // more than 8 ranges: batches of 8, each loaded at once, under a running
+      // maximum (a loop over the ranges, twice, waited a round trip apiece:
+      // 40 tokens on 12000 cached ones, 47 ranges, 39.0 -> 36.8 us a step)
       float M = -INFINITY;
-      for (int sp = 0; sp < ranges; ++sp) M = fmaxf(M, a.ml[(at0 + sp) * 2]);
-      for (int sp = 0; sp < ranges; ++sp) {
-        const float m = a.ml[(at0 + sp) * 2];
-        const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
-        const f32x4 p = *reinterpret_cast<const f32x4*>(a.part + (at0 + sp) * kPD + d);
+      for (int s0 = 0; s0 < ranges; s0 += 8) {
+        float2 x[8];
+        f32x4 p[8];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) O[e] += f * p[e];
-        L += f * a.ml[(at0 + sp) * 2 + 1];
+        for (int u = 0; u < 8; ++u) {  // past the last range: it again, unused
+          const int at = s0 + u < ranges ? s0 + u : ranges - 1;
+          x[u] = ml[at];
+          p[u] = *reinterpret_cast<const f32x4*>(part + (int64_t)at * kPD);
+        }
+        float mb = M;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) mb = fmaxf(mb, x[u].x);
+        const float alpha = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - mb);
+        L *= alpha;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) O[e] *= alpha;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if (s0 + u >= ranges) break;  // uniform
+          const float f = x[u].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(x[u].x - mb);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) O[e] += f * p[u][e];
+          L += f * x[u].y;
+        }
+        M = mb;
       }
     }
   }

@@ -139,6 +139,16 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     dense = rows * batch
     tiles = min(dense, tokens // PREFILL_Q_TILE + batch)
     least = PREFILL_SPLIT_MIN // PREFILL_KV_TILE
+    # half that for a few short workgroups (32 query tokens each) with CUs to
+    # spare, whose chain of key tiles is most of the launch: one prompt of 500
+    # tokens 22.1 -> 18.2 us, 619 on 95 cached ones 27.2 -> 24.6 us. With more
+    # ranges or more workgroups the merge costs it back (2 x 600 tokens 40.7 ->
+    # 42.2 us, 40 tokens on 12000 cached ones 39 -> 44 us).
+    fine = -(-2 * units // least)
+    half = PREFILL_Q_TILE // 2
+    few = min(-(-max_q // half) * batch, tokens // half + batch) * kv_heads * fine
+    if least < units and fine <= 8 and few <= cus // 2:
+        least //= 2
     fit = cus // max(1, dense * kv_heads)
     aim = max(least, -(-units // fit)) if fit else units
     if units <= least or aim <= PREFILL_DENSE_MAX:

@@ -108,7 +108,6 @@ PREFILL_SPLIT_MIN = 256        # keys per range at least
 PREFILL_DENSE_MAX = 6          # key tiles per range up to which a launch is not planned
 PREFILL_PLAN_SEQS = 1024       # sequences, and query tiles x KV heads, of a planned launch
 PREFILL_PLAN_TILES = 4096
-_prefill_ws: dict[torch.device, torch.Tensor] = {}
 _prefill_cu: dict[torch.device, int] = {}
 
 
@@ -209,12 +208,10 @@ def _prefill(q, k, v, page_table, cu_q, cu_k, lens_k, max_seqlen_q, softmax_scal
     elif splits > 1:
         ws_bytes = _lib.load().mkv_prefill_attention_workspace_bytes(Tq, Hq, splits)
     if ws_bytes > 0:
-        ws = _prefill_ws.get(dev)
-        if ws is None or ws.numel() < ws_bytes:
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            _prefill_ws[dev] = ws
-    # the workspace is reused by later calls on the stream: calls on one
-    # device must be issued on one stream (or be ordered by the caller)
+        # from torch's allocator at each call, which orders its reuse by stream:
+        # a plan or partial rows kept per device would be overwritten by a call
+        # on another stream while this one's kernels read them
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     fn = "mkv_prefill_attention_planned_bf16" if planned else "mkv_prefill_attention_bf16"
     _lib.call(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv,
               Hq, D, _lib.ptr(page_table), page_table.stride(0) if page_table is not None else 0,

@@ -410,3 +410,27 @@ def test_schedules_are_accepted(tokens, max_q, max_k, batch, heads):
                                                             splits) > 0
     elif splits > 1:
         assert split_len > 0 and split_len % 64 == 0 and splits * split_len >= max_k
+
+
+def test_planned_calls_on_two_streams():
+    """Calls of different lengths at once on two streams: neither reads the
+    other's plan or partial rows."""
+    case("attn_prefill: two streams, ragged prompts of different lengths")
+    jobs = []
+    for seed, lens in ((1, [1500, 90, 700, 2000] * 4), (2, [300, 2500, 64, 1100] * 4)):
+        g = torch.Generator().manual_seed(seed)
+        T = sum(lens)
+        q, k, v = (torch.randn(T, h, 256, generator=g).bfloat16().to(DEV) for h in (4, 1, 1))
+        cu = torch.tensor(np.cumsum([0] + lens), dtype=torch.int32, device=DEV)
+        want = A.attn_prefill(q, k, v, cu, cu, max(lens), max(lens))
+        jobs.append((torch.cuda.Stream(DEV), (q, k, v, cu, cu, max(lens), max(lens)), want, []))
+    torch.cuda.synchronize()
+    for _ in range(6):
+        for stream, args, _, outs in jobs:
+            with torch.cuda.stream(stream):
+                outs.append(A.attn_prefill(*args))
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    for _, _, want, outs in jobs:
+        for out in outs:
+            assert torch.equal(out.view(torch.int16), want.view(torch.int16))

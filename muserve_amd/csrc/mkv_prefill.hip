@@ -34,10 +34,10 @@
 // the time was which CU ran which tile: workgroups are dealt to the 8 XCDs in
 // turn, and with a sequence's tiles in consecutive workgroups an XCD had 113
 // key tiles on its fullest CU against 65 on average. With the order below
-// (prefill_attn_kernel) the same launch takes 254-262 us (1.05-1.08 PFLOP/s
-// of the visible pairs); six prompts of 80 to 4096 tokens, planned on the
-// device (prefill_plan_kernel), 177 -> 143 us. While a CU is busy its matrix
-// cores are so 59 % of the time, at 1.9 GHz.
+// (prefill_attn_kernel) the same launch takes 254-276 us (1.00-1.08 PFLOP/s
+// of the visible pairs, by the clock it gets); six prompts of 80 to 4096
+// tokens, planned on the device (prefill_plan_kernel), 177 -> 143 us. While a
+// CU is busy its matrix cores are so 59 % of the time, at 1.9 GHz.
 #include <float.h>
 #include <limits.h>
 #include <math.h>

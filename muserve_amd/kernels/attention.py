@@ -131,7 +131,7 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     device, which costs a launch of 7-8 us and pays for itself where that
     grid's ranges would be long or its sequences differ (MI355X: six prompts
     of 80 to 4096 tokens 177 -> 143 us; 8 equal prompts of 4096, where the
-    grid is balanced as it is, take 254-262 us without a plan).
+    grid is balanced as it is, take 254-276 us without a plan).
     """
     units = -(-max_k // PREFILL_KV_TILE)
     rows = -(-max_q // PREFILL_Q_TILE)

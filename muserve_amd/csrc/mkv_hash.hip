@@ -20,7 +20,7 @@
 // instructions per compression on the chain instead of about 1,550. It reads
 // the next block's K + W into registers before the rounds of this one, so no
 // LDS latency is left on the chain (64 prompts of up to 2560 tokens, a chain
-// of 320 compressions: 580 -> 564 us; 14 instructions of 4 cycles a round
+// of 320 compressions: 580 -> 556 us; 14 instructions of 4 cycles a round
 // bound it at 480 us).
 #include "mkv_device.h"
 
@@ -153,9 +153,9 @@ __global__ __launch_bounds__(kHashThreads) void block_hash_kernel(const uint8_t*
   // Iteration s: the rounds wave loads step s + 1's K + W (from buffer
   // (s + 1) & 1) and compresses step s from registers, while the schedule wave
   // fills step s + 2 (buffer s & 1, whose step the rounds wave holds since
-  // iteration s - 1, or from before the first); one barrier ends the iteration for both waves. Step u
-  // is block u % bpp of page u / bpp. Two iterations are unrolled, so that
-  // the two register sets swap by name.
+  // iteration s - 1, or from before the first); one barrier ends the iteration
+  // for both waves. Step u is block u % bpp of page u / bpp. Two iterations are
+  // unrolled, so that the two register sets swap by name.
   const int log_bpp = bpp - 1;
   auto iteration = [&](int64_t s, uint32_t (&now)[64], uint32_t (&after)[64])
                        __attribute__((always_inline)) {

@@ -19,9 +19,9 @@
 // first wave runs only the 64 rounds of each compression: about 900
 // instructions per compression on the chain instead of about 1,550. It reads
 // the next block's K + W into registers before the rounds of this one, so no
-// LDS latency is left on the chain (64 prompts of up to 2560 tokens, a chain
-// of 320 compressions: 580 -> 556 us; 14 instructions of 4 cycles a round
-// bound it at 480 us).
+// LDS latency is left on the chain (an admission of 64 prompts of up to 2560
+// tokens, whose hashes were 580 of its 763 us: 737 us; 14 instructions of 4
+// cycles a round bound the hashes at 480 us).
 #include "mkv_device.h"
 
 namespace mkv {

@@ -231,6 +231,11 @@ __device__ __forceinline__ void dma_wait() {
 // Keeps values derived from x out of registers held across the loop:
 // recomputing them costs a few instructions, holding them costs registers.
 __device__ __forceinline__ void opaque(uint32_t& x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void opaque(float& x) { asm volatile("" : "+v"(x)); }
+
+// The largest running maximum (absolute, log2 units) up to which a residue of
+// half an fp32 step, 2^-10, leaves the largest weight a bf16 1.
+constexpr float kFusedMax = 32768.f;
 
 // Instruction classes of __builtin_amdgcn_sched_group_barrier, and how many
 // matrix operands are read ahead of their use.
@@ -402,6 +407,7 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
       qb[s] = __builtin_bit_cast(bf16x8, ld16(row + 32 * s) ^ a.q_sign);
   }
   float m_run = -INFINITY, l_run = 0.f;  // l_run: this half wave's keys only
+  bool past_fused = false;  // uniform: some query's maximum is past kFusedMax
   f32x16 o[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -480,8 +486,10 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
       // to bf16: the error against float64 grew from 0.00205 to 0.00208.
       if (__builtin_amdgcn_ballot_w64(mx > m_run)) {
         const float m_new = fmaxf(m_run, mx);
-        const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
+        const float ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - ref);
         m_run = m_new;
+        past_fused = __builtin_amdgcn_ballot_w64(fabsf(ref) > kFusedMax) != 0;
         l_run *= alpha;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
@@ -489,6 +497,21 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
           for (int i = 0; i < 16; ++i) o[j][i] *= alpha;
       }
       const float m_ref = m_run == -INFINITY ? 0.f : m_run;  // a row with nothing seen yet
+      // The exponents below are fused, score * scale - m_ref, while m_ref is the
+      // rounded product: the largest score's exponent is that rounding's
+      // residue, at most half an fp32 step of m_ref. Up to kFusedMax its
+      // weight still rounds to a bf16 1. Past it (a step grows to more than
+      // the exponential's range) the products are rounded first, as m_ref was.
+      float mul = a.scale_log2;
+      if (__builtin_expect(past_fused, 0)) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+          float x = sq[i >> 4][i & 15] * a.scale_log2;
+          opaque(x);  // (or the product and the subtraction are fused again)
+          sq[i >> 4][i & 15] = x;
+        }
+        mul = 1.f;
+      }
       // O^T += V^T P^T in 16-key steps: half wave hf takes keys
       // 16 t + 4 hf .. +3 (elements 0-3) and 16 t + 8 + 4 hf .. +3. While the
       // matrix cores run step t, the vector unit makes step t + 1's
@@ -498,8 +521,8 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 8 * (t & 1) + 2 * i;
-          const float p0 = __builtin_amdgcn_exp2f(fmaf(sq[t >> 1][r], a.scale_log2, -m_ref));
-          const float p1 = __builtin_amdgcn_exp2f(fmaf(sq[t >> 1][r + 1], a.scale_log2, -m_ref));
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(sq[t >> 1][r], mul, -m_ref));
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(sq[t >> 1][r + 1], mul, -m_ref));
           l_run += p0 + p1;
           w[i] = bf16_pack(p0, p1);
         }

@@ -355,6 +355,31 @@ def test_query_tiles_scales_and_rising_maxima(lens, scale, grow):
     within(out, want)
 
 
+@pytest.mark.parametrize("lens", [[40, 97], [64] * 70 + [191, 320]])  # 4 and 8 waves
+@pytest.mark.parametrize("c", [300.0, 6000.0, 20500.0, 21500.0, -20500.0, 3e6])
+def test_large_finite_scores(c, lens):
+    """Scores far past 2^24 in log2 units, where one fp32 step is more than
+    the whole range of the exponential: the largest score's weight is still
+    exactly 1. Every query is c in every dim; the keys are |c| and |c| / 2 in
+    turn, so the visible keys of the larger product share the weight (the
+    other's is 0 in float64 too; sums of 256 products of 8-bit mantissas are
+    exact in fp32)."""
+    case(f"attn_prefill: finite scores of about {256 * c * abs(c):.1e}, {len(lens)} sequences")
+    g, cu = seqs(lens, 91)
+    T = int(cu[-1])
+    q = torch.full((T, 4, 256), c).bfloat16()
+    odd = torch.cat([torch.arange(n) for n in lens]) % 2
+    k = (abs(c) * (1.0 - 0.5 * odd))[:, None, None].expand(T, 1, 256).contiguous().bfloat16()
+    v = torch.randn(T, 1, 256, generator=g).bfloat16()
+    out = A.attn_prefill(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), cu.to(DEV), max(lens),
+                         max(lens))
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    want = att.prefill_attention(q.float().numpy(), k.float().numpy(), v.float().numpy(),
+                                 cu.numpy(), 256 ** -0.5, True, cu_k=cu.numpy(), stats=True)
+    within(out, want)
+
+
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("splits,heads,nqs,nks", [
     # both sides of the 64-query and 64-key tiles, no queries, no visible keys

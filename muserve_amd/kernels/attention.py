@@ -27,7 +27,6 @@ _DECODE_FNS = {torch.bfloat16: "mkv_decode_attention_bf16",
                torch.float16: "mkv_decode_attention_f16"}
 
 _errors: dict[torch.device, _lib.DeviceErrors] = {}
-_workspace: dict[torch.device, torch.Tensor] = {}
 
 
 def _errword(dev: torch.device) -> _lib.DeviceErrors:
@@ -41,6 +40,15 @@ def check_errors(device: torch.device | str = "cuda") -> None:
     dev = torch.device(device)
     if dev in _errors:
         _errors[dev].check("attn_decode")
+
+
+def _scratch(nbytes: int, dev: torch.device) -> torch.Tensor:
+    """A call's workspace, from torch's allocator at each call, which orders
+    its reuse by stream (and keeps it with the graph under capture). One buffer
+    kept per device would be overwritten by a call on another stream while
+    this one's kernels read it, and freed under them when a larger one is
+    needed."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=dev)
 
 
 def workspace_bytes(batch: int, num_kv_heads: int, num_q_heads: int, max_seqlen: int) -> int:
@@ -208,10 +216,7 @@ def _prefill(q, k, v, page_table, cu_q, cu_k, lens_k, max_seqlen_q, softmax_scal
     elif splits > 1:
         ws_bytes = _lib.load().mkv_prefill_attention_workspace_bytes(Tq, Hq, splits)
     if ws_bytes > 0:
-        # from torch's allocator at each call, which orders its reuse by stream:
-        # a plan or partial rows kept per device would be overwritten by a call
-        # on another stream while this one's kernels read them
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        ws = _scratch(ws_bytes, dev)
     fn = "mkv_prefill_attention_planned_bf16" if planned else "mkv_prefill_attention_bf16"
     _lib.call(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv,
               Hq, D, _lib.ptr(page_table), page_table.stride(0) if page_table is not None else 0,
@@ -286,14 +291,6 @@ def attn_decode_fp8(
                    cache_seqlens, page_table, softmax_scale, max_seqlen, out, shared_pages)
 
 
-def _workspace_for(dev, need):
-    ws = _workspace.get(dev)
-    if ws is None or ws.numel() < need:
-        ws = torch.empty(need, dtype=torch.uint8, device=dev)
-        _workspace[dev] = ws
-    return ws
-
-
 def _decode_contig(q, k_cache, v_cache, cache_seqlens, softmax_scale, max_seqlen, out):
     dev = _lib.require_gpu(q, k_cache, v_cache, cache_seqlens)
     B, one, Hq, D = q.shape
@@ -314,7 +311,7 @@ def _decode_contig(q, k_cache, v_cache, cache_seqlens, softmax_scale, max_seqlen
     if max_seqlen is None:
         max_seqlen = S
     scale = D ** -0.5 if softmax_scale is None else float(softmax_scale)
-    ws = _workspace_for(dev, workspace_bytes(B, Hkv, Hq, max_seqlen))
+    ws = _scratch(workspace_bytes(B, Hkv, Hq, max_seqlen), dev)
     _lib.call("mkv_decode_attention_contig", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
               1 if k_cache.dtype == torch.float16 else 0, Hkv, Hq, D, S,
               cache_seqlens.data_ptr(), B, int(min(max_seqlen, 1 << 24)), scale, out.data_ptr(),
@@ -349,9 +346,7 @@ def _decode(fn, q, k_cache, v_cache, k_scales, v_scales, cache_seqlens, page_tab
     elif out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
         raise ValueError("out must be a contiguous tensor shaped like q")
     scale = D ** -0.5 if softmax_scale is None else float(softmax_scale)
-    ws = _workspace_for(dev, workspace_bytes(B, Hkv, Hq, max_seqlen))
-    # the workspace is reused by later calls on the stream: calls on one
-    # device must be issued on one stream (or be ordered by the caller)
+    ws = _scratch(workspace_bytes(B, Hkv, Hq, max_seqlen), dev)
     scales = () if k_scales is None else (k_scales.data_ptr(), v_scales.data_ptr())
     if shared_pages < 0:
         raise ValueError("shared_pages must be >= 0")

@@ -98,6 +98,39 @@ def test_merge_of_few_pairs(lens):
     within_one_ulp(got, want)
 
 
+@pytest.mark.parametrize("contig", [False, True])
+def test_decode_on_two_streams(contig):
+    """Decode calls of different batches at once on two streams: neither reads
+    the other's prefix or pieces (few pairs of long contexts: every pair is cut
+    into many). The second stream's batch needs the larger workspace."""
+    case(f"decode attention on two streams, contiguous caches {contig}")
+    jobs = []
+    for seed, lens, Hq in ((61, [9000, 300, 7000], 4), (62, [2500, 8000, 100, 64, 6000], 8)):
+        if contig:
+            g = torch.Generator().manual_seed(seed)
+            q = torch.randn(len(lens), 1, Hq, 256, generator=g).bfloat16()
+            k, v = (torch.randn(len(lens), max(lens), Hq // 4, 256, generator=g).bfloat16()
+                    for _ in range(2))
+            table = None
+        else:
+            q, k, v, _, table = build(seed, lens, Hq, Hq // 4)
+            table = torch.from_numpy(table).to(DEV)
+        args = (q.to(DEV), k.to(DEV), v.to(DEV),
+                torch.tensor(lens, dtype=torch.int32, device=DEV), table)
+        want = A.attn_decode(*args)
+        jobs.append((torch.cuda.Stream(DEV), args, want, []))
+    torch.cuda.synchronize()
+    for _ in range(20):
+        for stream, args, _, outs in jobs:
+            with torch.cuda.stream(stream):
+                outs.append(A.attn_decode(*args))
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    for _, _, want, outs in jobs:
+        for out in outs:
+            assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
 def test_tight_bound_and_scale():
     lens = [300, 64, 511, 1]
     case(f"decode attention, max_seqlen 512 (no merge pass), scale 0.1, lens {lens}")

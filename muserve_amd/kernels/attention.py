@@ -113,7 +113,7 @@ def attn_prefill_paged(
 PREFILL_Q_TILE = 64            # query tokens per workgroup of the prefill kernel
 PREFILL_KV_TILE = 64           # keys per step of the prefill kernel (key ranges are multiples)
 PREFILL_SPLIT_MIN = 256        # keys per range at least
-PREFILL_DENSE_MAX = 6          # key tiles per range up to which a launch is not planned
+PREFILL_DENSE_MAX = 8          # key tiles per range up to which a launch is not planned
 PREFILL_PLAN_SEQS = 1024       # sequences, and query tiles x KV heads, of a planned launch
 PREFILL_PLAN_TILES = 4096
 _prefill_cu: dict[torch.device, int] = {}
@@ -137,20 +137,29 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     batch, in ranges of the same number of keys) does while it fits the CUs at
     once with short ranges; a planned launch sorts the tasks that exist on the
     device, which costs a launch of 7-8 us and pays for itself where that
-    grid's ranges would be long or its sequences differ (MI355X: six prompts
+    grid's ranges would be long and its sequences differ (MI355X: six prompts
     of 80 to 4096 tokens 177 -> 143 us; 8 equal prompts of 4096, where the
     grid is balanced as it is, take 254-276 us without a plan).
+
+    The line, PREFILL_DENSE_MAX, on 60 shapes (us without and with a plan): up
+    to 8 key tiles per range the grid was faster on all of them (8 chunks of 1
+    token on 5-16k cached ones 40, 51; 2 of 1 on 60k 73, 93; 500 tokens beside
+    31 x 50 31, 33); at 9 to 16 by the shape (1500 on 8k cached 61, 73; 6
+    prompts of 300 to 1250 45, 42; 4 of 250 to 1500 51, 42), but on all where
+    up to 8 sequences have one query tile each: a plan has little to sort and
+    more ranges to merge (2 x 1 on 120k 86, 114; 8 x 64 on 32k 69, 85).
     """
     units = -(-max_k // PREFILL_KV_TILE)
     rows = -(-max_q // PREFILL_Q_TILE)
     dense = rows * batch
     tiles = min(dense, tokens // PREFILL_Q_TILE + batch)
     least = PREFILL_SPLIT_MIN // PREFILL_KV_TILE
-    # half that for a few short workgroups (32 query tokens each) with CUs to
-    # spare, whose chain of key tiles is most of the launch: one prompt of 500
-    # tokens 22.1 -> 18.2 us, 619 on 95 cached ones 27.2 -> 24.6 us. With more
-    # ranges or more workgroups the merge costs it back (2 x 600 tokens 40.7 ->
-    # 42.2 us, 40 tokens on 12000 cached ones 39 -> 44 us).
+    # half of PREFILL_SPLIT_MIN for a few short workgroups (32 query tokens
+    # each) with CUs to spare, whose chain of key tiles is most of the launch:
+    # one prompt of 500 tokens 22.1 -> 18.2 us, 619 on 95 cached ones 27.2 ->
+    # 24.6 us. With more ranges or more workgroups the merge costs it back
+    # (2 x 600 tokens 40.7 -> 42.2 us, 40 tokens on 12000 cached ones 39 -> 44
+    # us).
     fine = -(-2 * units // least)
     half = PREFILL_Q_TILE // 2
     few = min(-(-max_q // half) * batch, tokens // half + batch) * kv_heads * fine
@@ -158,7 +167,8 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
         least //= 2
     fit = cus // max(1, dense * kv_heads)
     aim = max(least, -(-units // fit)) if fit else units
-    if units <= least or aim <= PREFILL_DENSE_MAX:
+    dense_max = PREFILL_DENSE_MAX * (2 if batch <= 8 and rows == 1 else 1)
+    if units <= least or aim <= dense_max:
         splits = max(1, -(-units // aim)) if fit else 1
         per = -(-units // splits)
         return (splits, per * PREFILL_KV_TILE, False) if splits > 1 else (1, 0, False)

@@ -17,6 +17,14 @@ def test_short_chunks_on_long_prefixes_take_the_grid(batch, max_q, max_k):
     assert 64 * 4 <= split_len <= 64 * 8 and splits * split_len >= max_k
 
 
+@pytest.mark.parametrize("max_q,max_k", [(1, 59467), (64, 59517), (64, 120000), (200, 16018)])
+def test_ranges_of_one_row_are_bounded(max_q, max_k):
+    """The merge walks a row's ranges serially: past 64 they get longer."""
+    splits, split_len, planned = prefill_schedule(max_q, max_q, max_k, 1, 1, True, CUS)
+    assert not planned and splits * split_len >= max_k
+    assert splits <= 64 or split_len >= 64 * 8
+
+
 def test_every_schedule_is_one_the_library_takes():
     """Over the range of sizes: workspace sizes exist, ranges cover the keys."""
     lib = _lib.load()

@@ -115,7 +115,7 @@ struct PrefillArgs {
   int32_t tok;           // query tokens per workgroup of this launch (a power of two)
   uint32_t ranks;        // query tiles of the longest sequence the launch covers
   uint32_t rank0;        // the first tile rank of this launch
-  int32_t turn;          // the grid is more than the CUs: ranks turn over the XCDs
+  int32_t turn;          // ranks turn over the XCDs
   int32_t splits;        // key ranges per (query tile, KV head) at most
   int32_t split_len;     // keys a range aims at (a multiple of the KV tile)
   Plan* plan;            // null: the grid is the schedule
@@ -282,9 +282,10 @@ __global__ __launch_bounds__(64 * WAVES) void prefill_attn_kernel(PrefillArgs a)
     // head, range) triples of a rank before the next rank. The dispatcher
     // hands consecutive workgroups to the 8 XCDs in turn, whatever their
     // load, so a triple moves one XCD on with every 8 workgroups: each XCD
-    // gets tiles of all ranks of every sequence. (A grid no larger than the
-    // CUs runs at once, in any order: no turn, and no divisions for it.
-    // Without the turn, sequences of 79, 76, 731 and 916 tokens took 42 us.)
+    // gets tiles of all ranks of every sequence. (Most grids no larger than
+    // the CUs, which run at once, do without: no divisions for it. In a larger
+    // one, sequences of 79, 76, 731 and 916 tokens took 28.4 us with the turn
+    // and 42 us without.)
     const uint32_t rank = a.rank0 + blockIdx.z;
     uint32_t at = blockIdx.x;
     b = blockIdx.y;
@@ -1108,7 +1109,16 @@ int prefill_attention(const char* fn, bool planned, const void* q, const void* k
   const int64_t triples = (int64_t)batch * num_kv_heads * splits;
   a.tok = small ? kQTok / 2 : kQTok;
   a.ranks = (uint32_t)ranks(a.tok);
-  a.turn = (int64_t)a.ranks * triples > kCus;
+  // Grids no larger than the CUs take their place from the grid, except where
+  // that puts each key range on one XCD and the later ranges have few of the
+  // tiles (causal prompts with no long prefix: the first range's XCD had 32
+  // tiles, the last one's 4). One prompt of 2000 tokens in 8 ranges 40.0 ->
+  // 34.5 us; on a long prefix every range has all tiles, and its keys are
+  // better read by one XCD (4 x 200 tokens on 3600 in 8 ranges 41.5 us, turned
+  // 43.9).
+  const bool uneven = splits % kXcds == 0 && causal &&
+                      2 * (int64_t)max_seqlen_q >= (int64_t)splits * split_len;
+  a.turn = (int64_t)a.ranks * triples > kCus || uneven;
   constexpr uint32_t kMaxZ = 65535;
   for (a.rank0 = 0; a.rank0 < a.ranks; a.rank0 += kMaxZ) {
     const dim3 grid((unsigned)(num_kv_heads * splits), (unsigned)batch,

@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "mkv_host.h"
 
 namespace {
@@ -25,6 +27,18 @@ int check_launch(const char* kernel) {
   if (e != hipSuccess)
     return set_error(MKV_E_LAUNCH, "%s: launch failed: %s", kernel, hipGetErrorString(e));
   return MKV_OK;
+}
+
+int device_cus() {
+  constexpr int kKept = 64;
+  static std::atomic<int> kept[kKept];
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  if (dev >= 0 && dev < kKept && (n = kept[dev].load(std::memory_order_relaxed)) > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+    return 256;
+  if (dev >= 0 && dev < kKept) kept[dev].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 }  // namespace mkv

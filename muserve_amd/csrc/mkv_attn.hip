@@ -55,7 +55,6 @@
 //     kernel merges them and also writes the zeros of empty pairs.
 #include <math.h>
 
-#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -1069,20 +1068,6 @@ template <int G, bool FP8>
 int occ_cap(int32_t pairs) {
   const int by_lds = (int)(kLdsPerCu / attn_lds_bytes<G, FP8>(pairs));
   return by_lds < 4 ? (by_lds < 1 ? 1 : by_lds) : 4;
-}
-
-// CUs of the current device (256, MI355X's count, when none can be queried),
-// asked once per device: a decode call needs the number four times.
-int device_cus() {
-  constexpr int kKept = 64;
-  static std::atomic<int> kept[kKept];
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (dev >= 0 && dev < kKept && (n = kept[dev].load(std::memory_order_relaxed)) > 0) return n;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    return 256;
-  if (dev >= 0 && dev < kKept) kept[dev].store(n, std::memory_order_relaxed);
-  return n;
 }
 
 template <int G, bool FP8, bool F16>

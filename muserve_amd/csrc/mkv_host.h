@@ -18,6 +18,10 @@ void clear_error();
 // Translates hipGetLastError() after a launch into MKV_OK / MKV_E_LAUNCH.
 int check_launch(const char* kernel);
 
+// CUs of the current device (256, MI355X's count, when none can be queried),
+// asked once per device: a decode call needs the number four times.
+int device_cus();
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
 

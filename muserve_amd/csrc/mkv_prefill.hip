@@ -73,7 +73,7 @@ constexpr int kWTok = 32;          // query tokens per wave
 constexpr int kQTok = 64;          // query tokens per workgroup of 8 waves
 constexpr int kKvTile = 64;        // KV tokens per step
 constexpr int kTileB = kKvTile * kPRow;     // bytes of one staged K (or V) tile
-constexpr int kCus = 256;          // MI355X; LDS holds one workgroup per CU
+constexpr int kCus = 256;          // MI355X's, the most a plan counts; LDS holds one workgroup per CU
 constexpr int kXcds = 8;           // MI355X: workgroups go round robin over 8 XCDs
 
 // One workgroup's task of a planned launch: range z of p of the query tile
@@ -116,6 +116,7 @@ struct PrefillArgs {
   uint32_t ranks;        // query tiles of the longest sequence the launch covers
   uint32_t rank0;        // the first tile rank of this launch
   int32_t turn;          // ranks turn over the XCDs
+  int32_t cus;           // the device's CUs (kCus at most)
   int32_t splits;        // key ranges per (query tile, KV head) at most
   int32_t split_len;     // keys a range aims at (a multiple of the KV tile)
   Plan* plan;            // null: the grid is the schedule
@@ -857,21 +858,24 @@ __global__ __launch_bounds__(THREADS) void prefill_plan_kernel(PrefillArgs a, in
     sum += red[w][0];
     most = red[w][1] > most ? red[w][1] : most;
   }
-  const uint64_t all = (uint64_t)(uint32_t)sum * (uint32_t)a.hkv;  // key tiles of all tasks
+  // key tiles of all tasks (the bounds on tiles and their keys keep it far
+  // below the clamp, which offsets that overlap could pass)
+  const uint64_t all64 = (uint64_t)(uint32_t)sum * (uint32_t)a.hkv;
+  const uint32_t all = all64 < (1u << 30) ? (uint32_t)all64 : 1u << 30, cus = (uint32_t)a.cus;
   // key tiles per range: no less than the key tiles per CU (so the tasks are
   // at most the query tiles and one more per CU) and than the launch's bound
-  int32_t least = (int32_t)((all + kCus - 1) / kCus);
+  int32_t least = (int32_t)((all + cus - 1) / cus);
   const int32_t bound = a.splits > 1 ? (most + a.splits - 1) / a.splits : most;
   least = least < bound ? bound : least;
   least = least < kPlanLeast ? kPlanLeast : least;
   int32_t cap = most;
   if (a.splits > 1 && least < most) {
-    cap = (int32_t)((all + all / 5 + kCus - 1) / kCus);
+    cap = (int32_t)((all + all / 5 + cus - 1) / cus);
     cap = cap < least ? least : cap > most ? most : cap;
     // kPlanTries candidates, evenly from the least to `far`
-    int32_t far = (int32_t)(all * 3 / (2 * kCus)) + 2;
+    int32_t far = (int32_t)(all * 3 / (2 * cus)) + 2;
     far = far < least ? least : far > most ? most : far;
-    if ((int64_t)tiles * a.hkv <= kCus) {  // (so tile_units holds them all)
+    if ((int64_t)tiles * a.hkv <= a.cus) {  // (so tile_units holds them all)
       const int32_t step = (far - least + kPlanTries - 1) / kPlanTries;
       for (int c = wave; c < kPlanTries; c += kWaves) {
         int32_t tried = least + c * (step > 1 ? step : 1);
@@ -880,7 +884,7 @@ __global__ __launch_bounds__(THREADS) void prefill_plan_kernel(PrefillArgs a, in
         for (int i = lane; i < tiles; i += 64) n += tile_ranges(tile_units[i], tried, a.splits);
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) n += __shfl_xor(n, d);
-        if (lane == 0 && (int64_t)n * a.hkv <= kCus) atomicMin(&found, tried);
+        if (lane == 0 && (int64_t)n * a.hkv <= a.cus) atomicMin(&found, tried);
       }
       __syncthreads();
       if (found != INT_MAX) cap = found;
@@ -1061,6 +1065,7 @@ int prefill_attention(const char* fn, bool planned, const void* q, const void* k
   a.out = static_cast<uint8_t*>(out);
   a.hkv = num_kv_heads;
   a.causal = causal ? 1 : 0;
+  a.cus = device_cus() < kCus ? device_cus() : kCus;
   a.splits = splits;
   a.split_len = splits > 1 && !planned ? split_len : INT_MAX / kKvTile * kKvTile;
   a.part = static_cast<float*>(workspace);
@@ -1105,7 +1110,7 @@ int prefill_attention(const char* fn, bool planned, const void* q, const void* k
   // waves, at most 240 with work).
   auto ranks = [&](int tok) { return (max_seqlen_q + (int64_t)tok - 1) / tok; };
   const int64_t dense = ranks(kQTok / 2) * batch, rows = num_q_tokens / (kQTok / 2) + batch;
-  const bool small = (dense < rows ? dense : rows) * num_kv_heads * splits <= kCus;
+  const bool small = (dense < rows ? dense : rows) * num_kv_heads * splits <= a.cus;
   const int64_t triples = (int64_t)batch * num_kv_heads * splits;
   a.tok = small ? kQTok / 2 : kQTok;
   a.ranks = (uint32_t)ranks(a.tok);
@@ -1118,7 +1123,7 @@ int prefill_attention(const char* fn, bool planned, const void* q, const void* k
   // 43.9).
   const bool uneven = splits % kXcds == 0 && causal &&
                       2 * (int64_t)max_seqlen_q >= (int64_t)splits * split_len;
-  a.turn = (int64_t)a.ranks * triples > kCus || uneven;
+  a.turn = (int64_t)a.ranks * triples > a.cus || uneven;
   constexpr uint32_t kMaxZ = 65535;
   for (a.rank0 = 0; a.rank0 < a.ranks; a.rank0 += kMaxZ) {
     const dim3 grid((unsigned)(num_kv_heads * splits), (unsigned)batch,

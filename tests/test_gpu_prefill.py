@@ -422,6 +422,149 @@ def test_planned_launches_pin_every_task(splits, heads, nqs, nks, causal):
     assert bool((out[Tq:] == 7.0).all())
 
 
+def _paged_one_hot(nks, heads, seed, spare=5, width=None):
+    """One-hot V rows (position j of a sequence is e_(j mod 256)) and random K
+    on shuffled pages: k, v pools and the block table, on the device."""
+    rng = np.random.default_rng(seed)
+    pages = [-(-n // 16) for n in nks]
+    P = sum(pages) + spare
+    perm = rng.permutation(P)
+    table = np.zeros((len(nks), width or max(1, max(pages))), dtype=np.int32)
+    v = torch.zeros(P, 16, heads, 256).bfloat16()
+    at = 0
+    for b, n in enumerate(pages):
+        table[b, :n] = perm[at:at + n]
+        v[torch.from_numpy(perm[at:at + n])] = _one_hot_keys(16 * n, heads).view(n, 16, heads, 256)
+        at += n
+    k = torch.randn(P, 16, heads, 256, generator=torch.Generator().manual_seed(seed)).bfloat16()
+    return k.to(DEV), v.to(DEV), torch.from_numpy(table).to(DEV)
+
+
+def _planned_paged(k, v, table, cu_q, lens_k, Tq, max_q, splits, causal=True):
+    """A planned launch over the pool through the C ABI, its workspace filled
+    with ones (NaN, if read as partial rows) and followed by a canary, as its
+    8 rows past Tq are: (out [Tq, 4 heads, 256], no canary touched)."""
+    heads, batch = k.shape[2], len(lens_k)
+    q = torch.zeros(Tq, 4 * heads, 256).bfloat16().to(DEV)
+    out = torch.full((Tq + 8, 4 * heads, 256), 7.0, dtype=torch.bfloat16, device=DEV)
+    n = _lib.load().mkv_prefill_attention_plan_bytes(Tq, 4 * heads, heads, batch, max_q, splits)
+    assert n > 0
+    ws = torch.full((n + 4096,), 0xFF, dtype=torch.uint8, device=DEV)
+    cu = torch.tensor(cu_q, dtype=torch.int32, device=DEV)
+    lens = torch.tensor(lens_k, dtype=torch.int32, device=DEV)
+    _lib.call("mkv_prefill_attention_planned_bf16", q.data_ptr(), k.data_ptr(), v.data_ptr(),
+              k.shape[0], heads, 4 * heads, 256, table.data_ptr(), table.stride(0),
+              table.shape[1], cu.data_ptr(), None, lens.data_ptr(), batch, Tq, max_q,
+              256 ** -0.5, int(causal), splits, out.data_ptr(), ws.data_ptr(), n,
+              A._errword(DEV).ptr(), _lib.stream_of(DEV))
+    torch.cuda.synchronize()
+    assert bool((ws[n:] == 0xFF).all()) and bool((out[Tq:] == 7.0).all())
+    return out[:Tq]
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("splits,heads,nqs,prefix", [
+    (12, 2, [300, 1, 0, 129, 64], [3000, 777, 50, 9, 1500]),  # all at once, ranges over 2 heads
+    (40, 1, [33, 65], [2527, 640]),                           # many ranges of few tiles
+    (3, 1, [1200, 700] + [70] * 220, [600, 0] + [100] * 220),  # more tasks than CUs
+    (4, 1, [500] + [20] * 300, [2000] + [30] * 300),          # more than 256 sequences
+    (9, 1, [500] + [0] * 280 + [20] * 19, [2000] + [30] * 299),  # and all tasks at once
+])
+def test_planned_paged_chunks_pin_every_task(splits, heads, nqs, prefix, causal):
+    """A planned launch over shuffled pages, with unequal chunks on unequal
+    cached prefixes: the schedule and the page lookups at every range's start."""
+    nks = [a + b for a, b in zip(nqs, prefix)]
+    case(f"prefill planned, paged: {len(nqs)} sequences, {heads} heads, {splits} ranges, "
+         f"causal={causal}")
+    k, v, table = _paged_one_hot(nks, heads, 44)
+    cu = np.cumsum([0] + nqs)
+    out = _planned_paged(k, v, table, cu, nks, int(cu[-1]), max(nqs), splits, causal)
+    A.check_errors(DEV)
+    for b, (nq, nk) in enumerate(zip(nqs, nks)):
+        want = _one_hot_want(nq, nk, causal)
+        for h in range(4 * heads):
+            if nq:
+                _bf16_close(out[cu[b]:cu[b + 1], h], want)
+
+
+def test_planned_paged_chunks_match_oracle():
+    """Random values through attn_prefill_paged, at a shape that it plans."""
+    chunk, prefix = [300, 40, 129], [3000, 500, 9000]
+    lens = [p + c for p, c in zip(prefix, chunk)]
+    case(f"attn_prefill_paged planned: prefix {prefix} chunk {chunk}")
+    assert A.prefill_schedule(sum(chunk), max(chunk), max(lens), 3, 1, True,
+                              A._prefill_cus(torch.device(DEV)))[2]
+    g = torch.Generator().manual_seed(45)
+    k, _, table = _paged_one_hot(lens, 1, 45)
+    v = torch.randn(k.shape, generator=g).bfloat16().to(DEV)
+    cu = torch.tensor(np.cumsum([0] + chunk), dtype=torch.int32)
+    q = torch.randn(sum(chunk), 4, 256, generator=g).bfloat16()
+    seq_lens = torch.tensor(lens, dtype=torch.int32)
+    out = A.attn_prefill_paged(q.to(DEV), k, v, cu.to(DEV), seq_lens.to(DEV), table, max(chunk),
+                               max_seqlen_k=max(lens))
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    want = att.prefill_attention(q.float().numpy(), k.float().cpu().numpy(),
+                                 v.float().cpu().numpy(), cu.numpy(), 256 ** -0.5, True,
+                                 lens_k=seq_lens.numpy(), page_table=table.cpu().numpy(),
+                                 stats=True)
+    within(out, want)
+
+
+@pytest.mark.parametrize("what", ["page", "length", "negative length", "queries", "decreasing",
+                                  "overlapping"])
+def test_planned_launches_flag_bad_inputs(what):
+    """Ids, lengths and offsets that the plan kernel (or a planned range)
+    finds outside their buffers are flagged; the other sequences are served and
+    nothing is written outside the queries, the output or the workspace."""
+    case(f"prefill planned, paged: bad {what}")
+    nqs, nks, splits = [100, 200, 70], [1500, 900, 640], 8
+    k, v, table = _paged_one_hot(nks, 1, 46)
+    cu, lens, Tq, max_q = list(np.cumsum([0] + nqs)), list(nks), sum(nqs), max(nqs)
+    served = {0: (0, nqs[0], nks[0]), 1: (100, nqs[1], nks[1]), 2: (300, nqs[2], nks[2])}
+    text = "table"
+    if what == "page":
+        table[1, 20] = k.shape[0] + 3  # keys 320 .. 335 of sequence 1 read as zeros
+        text = "page id"
+        del served[1]
+    elif what == "length":  # 200 keys past the table's 94 pages: clamped to them
+        lens[0] = 16 * table.shape[1] + 200
+        served[0] = (0, nqs[0], 16 * table.shape[1])
+    elif what == "negative length":
+        lens[2] = -5
+        del served[2]
+    elif what == "queries":  # the last sequence would end 10 rows past the buffer
+        cu[3] += 10
+        del served[2]
+    elif what == "decreasing":  # sequence 1 ends before it begins, 2 is empty
+        cu[2] = cu[3] = 60
+        del served[1], served[2]
+    else:  # the same rows and keys four times: more tiles than the bounds expect
+        nqs, nks = [640], [1500]
+        cu, Tq, max_q = [0, 640, 0, 640, 0, 640, 0, 640], 640, 640
+        lens, table = [1500] * 7, table[:1].expand(7, -1).contiguous()
+        served = {}
+    out = _planned_paged(k, v, table, cu, lens, Tq, max_q, splits)
+    with pytest.raises(_lib.MkvDeviceError, match=text):
+        A.check_errors(DEV)
+    for first, nq, nk in served.values():
+        want = _one_hot_want(nq, nk, True)
+        for h in range(4):
+            _bf16_close(out[first:first + nq, h], want)
+    if what == "queries":
+        assert bool((out[300:] == 7.0).all())
+    elif what == "decreasing":
+        assert bool((out[100:] == 7.0).all())
+    elif what == "negative length":
+        assert not out[300:].float().abs().sum().item()  # no key: zeros
+    elif what == "page":  # each key's weight is 1 / n; those of the bad page count nothing
+        want = _one_hot_want(200, 900, True)
+        n = np.arange(701, 901)[:, None]
+        want[:, 320 % 256:320 % 256 + 16] -= 1.0 / n
+        for h in range(4):
+            _bf16_close(out[100:300, h], want)
+
+
 @pytest.mark.parametrize("tokens,max_q,max_k,batch,heads", [
     (1, 1, 1, 1, 1), (77, 77, 77, 1, 1), (13897, 4096, 4096, 6, 1), (32768, 4096, 4096, 8, 1),
     (2572, 1428, 6540, 2, 1), (3, 1, 1 << 20, 3, 2), (4096, 16, 64, 256, 1),

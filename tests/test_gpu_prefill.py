@@ -580,6 +580,26 @@ def test_schedules_are_accepted(tokens, max_q, max_k, batch, heads):
         assert split_len > 0 and split_len % 64 == 0 and splits * split_len >= max_k
 
 
+@pytest.mark.parametrize("lens", [[64], [40, 64, 7], [300, 20]])
+def test_loose_bounds_cost_no_plan(lens, monkeypatch):
+    """Bounds far above what the rows can hold: the schedule is made for the
+    rows, and the output is that of tight bounds."""
+    case(f"attn_prefill lens {lens} under bounds of 4096")
+    g, cu = seqs(lens, 47)
+    T = int(cu[-1])
+    q, k, v = (torch.randn(T, h, 256, generator=g).bfloat16().to(DEV) for h in (4, 1, 1))
+    cu = cu.to(DEV)
+    made = []
+    rule = A.prefill_schedule
+    monkeypatch.setattr(A, "prefill_schedule", lambda *a: made.append(rule(*a)) or made[-1])
+    got = A.attn_prefill(q, k, v, cu, cu, 4096, 4096)
+    want = A.attn_prefill(q, k, v, cu, cu, T, T)
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    assert made[0] == made[1] and not made[0][2]
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def test_planned_calls_on_two_streams():
     """Calls of different lengths at once on two streams: neither reads the
     other's plan or partial rows."""

@@ -230,23 +230,34 @@ def _prefill(q, k, v, page_table, cu_q, cu_k, lens_k, max_seqlen_q, softmax_scal
     max_k = int(max_seqlen_k) if max_seqlen_k is not None else page_table.shape[1] * 16
     if page_table is None:
         max_k = min(max_k, units)
-    splits, split_len, planned = prefill_schedule(Tq, max_q, max_k, batch, Hkv, causal,
-                                                  _prefill_cus(dev))
+    # a plan holds PREFILL_PLAN_SEQS sequences: more of them are planned so many
+    # at a time (1500 tokens beside 2000 x 16: one launch of 48000 workgroups,
+    # nearly all empty, took 252 us)
+    some = min(batch, PREFILL_PLAN_SEQS)
+    sched = prefill_schedule(Tq, max_q, max_k, some, Hkv, causal, _prefill_cus(dev))
+    if not sched[2] and some < batch:
+        some = batch
+        sched = prefill_schedule(Tq, max_q, max_k, batch, Hkv, causal, _prefill_cus(dev))
+    splits, split_len, planned = sched
     ws, ws_bytes = None, 0
     if planned:
-        ws_bytes = _lib.load().mkv_prefill_attention_plan_bytes(Tq, Hq, Hkv, batch, max_q,
-                                                                splits)
+        ws_bytes = _lib.load().mkv_prefill_attention_plan_bytes(Tq, Hq, Hkv, some, max_q, splits)
     elif splits > 1:
         ws_bytes = _lib.load().mkv_prefill_attention_workspace_bytes(Tq, Hq, splits)
     if ws_bytes > 0:
         ws = _scratch(ws_bytes, dev)
     fn = "mkv_prefill_attention_planned_bf16" if planned else "mkv_prefill_attention_bf16"
-    _lib.call(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv,
-              Hq, D, _lib.ptr(page_table), page_table.stride(0) if page_table is not None else 0,
-              page_table.shape[1] if page_table is not None else 0, cu_q.data_ptr(),
-              _lib.ptr(cu_k), _lib.ptr(lens_k), batch, Tq, max_q, scale,
-              1 if causal else 0, splits, *(() if planned else (split_len,)), out.data_ptr(),
-              _lib.ptr(ws), ws_bytes, _errword(dev).ptr(), _lib.stream_of(dev))
+    stride, width = (page_table.stride(0), page_table.shape[1]) if page_table is not None else (0, 0)
+
+    def row(t, i):  # of an int32 tensor
+        return None if t is None else t.data_ptr() + 4 * i
+
+    for b in range(0, max(batch, 1), max(some, 1)):
+        _lib.call(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv, Hq, D,
+                  row(page_table, b * stride), stride, width, row(cu_q, b), row(cu_k, b),
+                  row(lens_k, b), min(some, batch - b), Tq, max_q, scale, 1 if causal else 0,
+                  splits, *(() if planned else (split_len,)), out.data_ptr(), _lib.ptr(ws),
+                  ws_bytes, _errword(dev).ptr(), _lib.stream_of(dev))
     return out
 
 

@@ -580,6 +580,35 @@ def test_schedules_are_accepted(tokens, max_q, max_k, batch, heads):
         assert split_len > 0 and split_len % 64 == 0 and splits * split_len >= max_k
 
 
+@pytest.mark.parametrize("paged", [False, True])
+def test_more_sequences_than_a_plan_holds(paged, monkeypatch):
+    """Ragged batches of more than 1024 sequences are planned 1024 at a time,
+    whichever part the long ones are in."""
+    lens = [3] * 1024 + [700] + [2] * 1100 + [300]
+    case(f"attn_prefill {len(lens)} sequences of 2..700, paged={paged}")
+    cu = np.cumsum([0] + lens)
+    T = int(cu[-1])
+    q = torch.zeros(T, 4, 256).bfloat16().to(DEV)
+    cu_d = torch.tensor(cu, dtype=torch.int32, device=DEV)
+    calls = []
+    real = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: calls.append(name) or real(name, *a))
+    if paged:
+        k, v, table = _paged_one_hot(lens, 1, 48)
+        out = A.attn_prefill_paged(q, k, v, cu_d, torch.tensor(lens, dtype=torch.int32, device=DEV),
+                                   table, max(lens), max_seqlen_k=max(lens))
+    else:
+        v = torch.cat([_one_hot_keys(n) for n in lens]).to(DEV)
+        k = torch.randn(T, 1, 256, generator=torch.Generator().manual_seed(48)).bfloat16().to(DEV)
+        out = A.attn_prefill(q, k, v, cu_d, cu_d, max(lens), max(lens))
+    torch.cuda.synchronize()
+    A.check_errors(DEV)
+    assert calls == ["mkv_prefill_attention_planned_bf16"] * 3
+    want = np.concatenate([_one_hot_want(n, n, True) for n in lens])
+    for h in range(4):
+        _bf16_close(out[:, h], want)
+
+
 @pytest.mark.parametrize("lens", [[64], [40, 64, 7], [300, 20]])
 def test_loose_bounds_cost_no_plan(lens, monkeypatch):
     """Bounds far above what the rows can hold: the schedule is made for the

@@ -178,6 +178,13 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     if units <= least or aim <= dense_max:
         splits = max(1, -(-units // aim)) if fit else 1
         per = -(-units // splits)
+        # without a causal mask every row has all the ranges: they have to save
+        # more key tiles (2.4 us each) than the merge of their partial rows
+        # costs (8 x 300 tokens 22.2 us in one range, 28.6 in two; 8 x 500 31.3,
+        # 33.9; 4 x 700 in one 38.6, in three 33.5)
+        merge_us = 4 + splits * tokens * 4 * kv_heads * 2064 / 8e6
+        if not causal and (units - per) * 2.4 < merge_us:
+            return 1, 0, False
         return (splits, per * PREFILL_KV_TILE, False) if splits > 1 else (1, 0, False)
     mean = units - (min(rows, units) - 1) / 2 if causal else units
     share = tiles * kv_heads * mean / cus  # key tiles per CU, at most

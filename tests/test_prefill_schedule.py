@@ -25,6 +25,13 @@ def test_ranges_of_one_row_are_bounded(max_q, max_k):
     assert splits <= 64 or split_len >= 64 * 8
 
 
+@pytest.mark.parametrize("batch,n,one", [(8, 300, True), (8, 500, True), (4, 300, True),
+                                         (4, 700, False), (1, 300, False), (1, 2000, False)])
+def test_ranges_without_a_mask_pay_for_their_merge(batch, n, one):
+    splits, _, planned = prefill_schedule(batch * n, n, n, batch, 1, False, CUS)
+    assert not planned and (splits == 1) == one
+
+
 def test_every_schedule_is_one_the_library_takes():
     """Over the range of sizes: workspace sizes exist, ranges cover the keys."""
     lib = _lib.load()

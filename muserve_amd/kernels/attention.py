@@ -151,6 +151,8 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     more ranges to merge (2 x 1 on 120k 86, 114; 8 x 64 on 32k 69, 85).
     """
     units = -(-max_k // PREFILL_KV_TILE)
+    if units <= PREFILL_SPLIT_MIN // PREFILL_KV_TILE:
+        return 1, 0, False
     rows = -(-max_q // PREFILL_Q_TILE)
     dense = rows * batch
     tiles = min(dense, tokens // PREFILL_Q_TILE + batch)
@@ -175,15 +177,14 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     fit = cus // max(1, dense * kv_heads)
     aim = max(least, -(-units // fit)) if fit else units
     dense_max = PREFILL_DENSE_MAX * (2 if batch <= 8 and rows == 1 else 1)
-    if units <= least or aim <= dense_max:
+    if aim <= dense_max:
         splits = max(1, -(-units // aim)) if fit else 1
         per = -(-units // splits)
         # without a causal mask every row has all the ranges: they have to save
         # more key tiles (2.4 us each) than the merge of their partial rows
         # costs (8 x 300 tokens 22.2 us in one range, 28.6 in two; 8 x 500 31.3,
         # 33.9; 4 x 700 in one 38.6, in three 33.5)
-        merge_us = 4 + splits * tokens * 4 * kv_heads * 2064 / 8e6
-        if not causal and (units - per) * 2.4 < merge_us:
+        if not causal and (units - per) * 2.4 < 4 + splits * tokens * 4 * kv_heads * 2064 / 8e6:
             return 1, 0, False
         return (splits, per * PREFILL_KV_TILE, False) if splits > 1 else (1, 0, False)
     mean = units - (min(rows, units) - 1) / 2 if causal else units
@@ -233,18 +234,21 @@ def _prefill(q, k, v, page_table, cu_q, cu_k, lens_k, max_seqlen_q, softmax_scal
     # bounds that the rows already give: a caller's loose ones would buy a plan
     # and empty workgroups (one prompt of 64 tokens under bounds of 4096: 17.9
     # us, 11.0 under its own)
-    max_q = min(int(max_seqlen_q), Tq)
+    max_q = min(int(max_seqlen_q), max(Tq, 1))  # (no rows: refused below)
     max_k = int(max_seqlen_k) if max_seqlen_k is not None else page_table.shape[1] * 16
     if page_table is None:
         max_k = min(max_k, units)
-    # a plan holds PREFILL_PLAN_SEQS sequences: more of them are planned so many
-    # at a time (1500 tokens beside 2000 x 16: one launch of 48000 workgroups,
-    # nearly all empty, took 252 us)
-    some = min(batch, PREFILL_PLAN_SEQS)
-    sched = prefill_schedule(Tq, max_q, max_k, some, Hkv, causal, _prefill_cus(dev))
-    if not sched[2] and some < batch:
-        some = batch
-        sched = prefill_schedule(Tq, max_q, max_k, batch, Hkv, causal, _prefill_cus(dev))
+    sched = prefill_schedule(Tq, max_q, max_k, min(batch, PREFILL_PLAN_SEQS), Hkv, causal,
+                             _prefill_cus(dev))
+    some = batch
+    if batch > PREFILL_PLAN_SEQS:
+        # more than a plan holds are planned so many at a time (1500 tokens
+        # beside 2000 x 16: one launch of 48000 workgroups, nearly all empty,
+        # took 252 us)
+        if sched[2] and batch <= 65535:  # (the library's limit for one call)
+            some = PREFILL_PLAN_SEQS
+        else:
+            sched = prefill_schedule(Tq, max_q, max_k, batch, Hkv, causal, _prefill_cus(dev))
     splits, split_len, planned = sched
     ws, ws_bytes = None, 0
     if planned:
@@ -254,18 +258,25 @@ def _prefill(q, k, v, page_table, cu_q, cu_k, lens_k, max_seqlen_q, softmax_scal
     if ws_bytes > 0:
         ws = _scratch(ws_bytes, dev)
     fn = "mkv_prefill_attention_planned_bf16" if planned else "mkv_prefill_attention_bf16"
-    stride, width = (page_table.stride(0), page_table.shape[1]) if page_table is not None else (0, 0)
-
-    def row(t, i):  # of an int32 tensor
-        return None if t is None else t.data_ptr() + 4 * i
-
-    for b in range(0, max(batch, 1), max(some, 1)):
-        _lib.call(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv, Hq, D,
-                  row(page_table, b * stride), stride, width, row(cu_q, b), row(cu_k, b),
-                  row(lens_k, b), min(some, batch - b), Tq, max_q, scale, 1 if causal else 0,
-                  splits, *(() if planned else (split_len,)), out.data_ptr(), _lib.ptr(ws),
-                  ws_bytes, _errword(dev).ptr(), _lib.stream_of(dev))
-    return out
+    table, stride, width = None, 0, 0
+    if page_table is not None:
+        table, stride, width = page_table.data_ptr(), page_table.stride(0), page_table.shape[1]
+    cu_qp, cu_kp, lens_kp = cu_q.data_ptr(), _lib.ptr(cu_k), _lib.ptr(lens_k)
+    first = 0
+    while True:
+        _lib.call(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), units, Hkv, Hq, D, table, stride,
+                  width, cu_qp, cu_kp, lens_kp, min(some, batch - first), Tq, max_q, scale,
+                  1 if causal else 0, splits, *(() if planned else (split_len,)), out.data_ptr(),
+                  _lib.ptr(ws), ws_bytes, _errword(dev).ptr(), _lib.stream_of(dev))
+        first += some
+        if first >= batch:
+            return out
+        cu_qp += 4 * some  # (int32 offsets, lengths and page ids)
+        if table is None:
+            cu_kp += 4 * some
+        else:
+            table += 4 * some * stride
+            lens_kp += 4 * some
 
 
 def attn_decode(

@@ -195,6 +195,16 @@ def test_bad_page_and_bad_offsets_are_flagged():
         A.check_errors(DEV)
 
 
+def test_offsets_without_rows_are_refused():
+    case("attn_prefill with no query rows and an offset past them")
+    q = torch.empty(0, 4, 256, dtype=torch.bfloat16, device=DEV)
+    k = torch.zeros(20, 1, 256, dtype=torch.bfloat16, device=DEV)
+    cu_q = torch.tensor([0, 5], dtype=torch.int32, device=DEV)
+    cu_k = torch.tensor([0, 20], dtype=torch.int32, device=DEV)
+    with pytest.raises(_lib.MkvError, match="null pointer"):
+        A.attn_prefill(q, k, k.clone(), cu_q, cu_k, 5, 20)
+
+
 @pytest.mark.parametrize("split_len", [64, 128, 192])
 def test_forced_key_splits_through_the_c_abi(split_len):
     """Key ranges of one, two and three 64-key tiles (the double-buffered

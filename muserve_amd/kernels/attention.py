@@ -15,7 +15,7 @@ word that ``check_errors(device)`` raises.
 """
 from __future__ import annotations
 
-import math
+import functools
 
 import torch
 
@@ -57,6 +57,19 @@ def workspace_bytes(batch: int, num_kv_heads: int, num_q_heads: int, max_seqlen:
     if n < 0:
         raise ValueError("bad attention shape")
     return n
+
+
+@functools.lru_cache(maxsize=1024)
+def _decode_bytes(batch: int, num_kv_heads: int, num_q_heads: int, dev: torch.device) -> int:
+    return workspace_bytes(batch, num_kv_heads, num_q_heads, 0)
+
+
+def _decode_scratch(B: int, Hkv: int, Hq: int, max_seqlen: int, dev: torch.device) -> torch.Tensor:
+    """The size depends on the shape and the device alone (asking the library
+    again costs a decode call 1 us, as much as the allocation)."""
+    if max_seqlen < 0:
+        raise ValueError("bad attention shape")
+    return _scratch(_decode_bytes(B, Hkv, Hq, dev), dev)
 
 
 def attn_prefill(
@@ -363,7 +376,7 @@ def _decode_contig(q, k_cache, v_cache, cache_seqlens, softmax_scale, max_seqlen
     if max_seqlen is None:
         max_seqlen = S
     scale = D ** -0.5 if softmax_scale is None else float(softmax_scale)
-    ws = _scratch(workspace_bytes(B, Hkv, Hq, max_seqlen), dev)
+    ws = _decode_scratch(B, Hkv, Hq, max_seqlen, dev)
     _lib.call("mkv_decode_attention_contig", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
               1 if k_cache.dtype == torch.float16 else 0, Hkv, Hq, D, S,
               cache_seqlens.data_ptr(), B, int(min(max_seqlen, 1 << 24)), scale, out.data_ptr(),
@@ -398,7 +411,7 @@ def _decode(fn, q, k_cache, v_cache, k_scales, v_scales, cache_seqlens, page_tab
     elif out.shape != q.shape or out.dtype != q.dtype or not out.is_contiguous():
         raise ValueError("out must be a contiguous tensor shaped like q")
     scale = D ** -0.5 if softmax_scale is None else float(softmax_scale)
-    ws = _scratch(workspace_bytes(B, Hkv, Hq, max_seqlen), dev)
+    ws = _decode_scratch(B, Hkv, Hq, max_seqlen, dev)
     scales = () if k_scales is None else (k_scales.data_ptr(), v_scales.data_ptr())
     if shared_pages < 0:
         raise ValueError("shared_pages must be >= 0")

@@ -983,7 +983,7 @@ def run_prefix(steps: int, warmup: int, with_cpu: bool) -> dict:
         "roofline": {"kernels": [
             {"kernel": "block_hash_kernel (mkv_block_hash_sha256)", "bound": "integer ALU / latency",
              "note": "the longest request's chain of SHA-256 rounds (two compressions per "
-                     "page, ~944 instructions each); no HBM roofline claim",
+                     "page, ~900 instructions each); no HBM roofline claim",
              "launch_ms": round(hash_ms, 3),
              "GB_hashed_per_s": round(8 * int(cu_t[-1]) / (hash_ms / 1e3) / 1e9, 3)},
             {"kernel": "mkv_bm_step (release run, speculation, group and step kernels)",

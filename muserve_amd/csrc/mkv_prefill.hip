@@ -36,7 +36,7 @@
 // key tiles on its fullest CU against 65 on average. With the order below
 // (prefill_attn_kernel) the same launch takes 254-276 us (1.00-1.08 PFLOP/s
 // of the visible pairs, by the clock it gets); six prompts of 80 to 4096
-// tokens, planned on the device (prefill_plan_kernel), 177 -> 143 us. While a
+// tokens, planned on the device (prefill_plan_kernel), 177 -> 142-149 us. While a
 // CU is busy its matrix cores are so 59 % of the time, at 1.9 GHz.
 #include <float.h>
 #include <limits.h>
@@ -218,7 +218,9 @@ __device__ __forceinline__ int32_t units_of(int64_t keys) {
 // 16 bytes per lane from base + voff into LDS at lds + 16 * lane. Issued from
 // inline assembly: the compiler neither waits for it nor moves LDS accesses
 // across it; the waits are explicit (dma_wait before the tile's barrier). M0
-// holds the destination; nothing else in this file uses M0.
+// holds the destination; nothing else in this file uses M0 (to the compiler a
+// reserved register, which it writes only right before an instruction that
+// reads it and refuses in a clobber list).
 __device__ __forceinline__ void dma16(const uint8_t* base, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :
@@ -758,11 +760,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 //     far above the key tiles per CU (1.5 times + 2);
 //   * else 1.2 times the key tiles per CU: the longest tasks start first, and
 //     the shorter ones fill the CUs as they come free.
-// Only the lengths on the device say which, and a grid sized on the host has
-// workgroups with nothing to do among the others, which leaves some XCD with
-// more tasks than CUs (two 1.3k-token chunks on 3-5k tokens: attention kernel
-// 107 us with a dense grid of 7 ranges, 64 us planned; sorted by length alone,
-// without the XCDs' grouping, 66 us). The plan takes 7-8 us.
+// Only the lengths on the device say which; a grid sized on the host cuts all
+// sequences as the longest, or not at all. Whole calls, planned and with the
+// best such grid of at most one task per CU: 6 prompts of 190 to 2180 tokens
+// 50 and 107 us, 4 of 400 to 2280 52 and 113, two chunks of 1.0-1.4k on 3-6k
+// tokens 84 and 83 (the rule in prefill_schedule draws the line). Sorted by
+// length alone, without the XCDs' grouping, those chunks' attention took 66 us
+// instead of 64. The plan takes 7-9 us.
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void prefill_plan_kernel(PrefillArgs a, int32_t batch) {
   __shared__ int32_t pre[THREADS];          // the sequences' first tiles

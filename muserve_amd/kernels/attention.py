@@ -157,11 +157,11 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
 
     The line, PREFILL_DENSE_MAX, on 60 shapes (us without and with a plan): up
     to 8 key tiles per range the grid was faster on all of them (8 chunks of 1
-    token on 5-16k cached ones 40, 51; 2 of 1 on 60k 73, 93; 500 tokens beside
-    31 x 50 31, 33); at 9 to 16 by the shape (1500 on 8k cached 61, 73; 6
-    prompts of 300 to 1250 45, 42; 4 of 250 to 1500 51, 42), but on all where
+    token on 6-14k cached ones 40, 51; 2 of 1 on 60k 73, 93; 500 tokens beside
+    31 x 50 31, 33); at 9 to 16 by the shape (1200 on 7k cached 61, 73; 6
+    prompts of 360 to 1240 45, 42; 4 of 265 to 1520 51, 42), but on all where
     up to 8 sequences have one query tile each: a plan has little to sort and
-    more ranges to merge (2 x 1 on 120k 86, 114; 8 x 64 on 32k 69, 85).
+    more ranges to merge (2 x 1 on up to 120k 86, 114; 8 x 64 on up to 32k 69, 85).
     """
     units = -(-max_k // PREFILL_KV_TILE)
     if units <= PREFILL_SPLIT_MIN // PREFILL_KV_TILE:
@@ -173,7 +173,7 @@ def prefill_schedule(tokens: int, max_q: int, max_k: int, batch: int, kv_heads: 
     # twice that where a row would have more than PREFILL_RANGES ranges: the
     # merge walks them 8 at a time, about 0.3 us a range against 2.4 us a key
     # tile (64 tokens on 60000 cached ones in 235 ranges 108 us, in 118 76 us;
-    # on 16000 in 63 or in 32 the same)
+    # 200 on 16000 in 58, 46 or 23 ranges 48, 46 and 51 us)
     if units > PREFILL_RANGES * least:
         least *= 2
     # half of PREFILL_SPLIT_MIN for a few short workgroups (32 query tokens
